@@ -1,8 +1,9 @@
 """Ahead-of-time build of librq.so for gfx950.
 
 1. hipcc --genco compiles each kernel source (csrc/rq_kernels.hip: the Q8_1
-   pass and the dot4 matvecs; csrc/rq_mmq.hip: the int8-MFMA matvecs) into
-   one gfx950 code object each.
+   pass and the dot4 matvecs; csrc/rq_mmq.hip: the int8-MFMA matvecs;
+   csrc/rq_cols.hip: the matvecs over 4 to 64 columns) into one gfx950 code
+   object each.
 2. An assembler stub (.incbin) embeds the code objects in the library.
 3. hipcc compiles csrc/rq_static.hip (the fixed device scratch of
    rq_matmul_many_noalloc) as an ordinary host + device object.
@@ -36,7 +37,7 @@ TIMELINE_LIB = os.path.join(LIBDIR, "librq_tl.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 ARCH = "gfx950"
 # Kernel sources, one code object each (embedded as <name>_blob).
-KERNEL_SOURCES = ("rq_kernels", "rq_mmq")
+KERNEL_SOURCES = ("rq_kernels", "rq_mmq", "rq_cols")
 
 # Device code: IEEE-correct f32 division (the Q8_1 scale and codes must match
 # the CPU bit for bit) and no packed-f32 instructions (they have given wrong

@@ -30,6 +30,7 @@
 
 extern "C" const unsigned char rq_kernels_blob[];  // rq_kernels.hip: Q8_1 pass, dot4 matvecs
 extern "C" const unsigned char rq_mmq_blob[];      // rq_mmq.hip: int8-MFMA matvecs
+extern "C" const unsigned char rq_cols_blob[];     // rq_cols.hip: matvecs over 4 to 64 columns
 // rq_static.hip: the device address of the fixed scratch of
 // rq_matmul_many_noalloc on the current device.
 extern "C" __attribute__((visibility("hidden"))) hipError_t rq_noalloc_scratch(int device, void** ptr, size_t* bytes);
@@ -245,7 +246,7 @@ struct rq_ctx {
     hipFunction_t mmq[RQ_NUM_FMTS + 1][3][3] = {};
     hipFunction_t mmqf[RQ_NUM_FMTS + 1][3] = {};
     hipFunction_t mmqd[RQ_NUM_FMTS][3][3] = {};
-    hipFunction_t mmqg[RQ_NUM_FMTS + 1][4][3] = {};  // 8 x G columns, G = 2, 4 (Q6_K also 6, 8)
+    hipFunction_t mmqg[RQ_NUM_FMTS + 1][2][3] = {};  // 8 x G columns, G = 2, 4 (Q6_K and the mix: 2)
     // 16 x G columns with four-activation entries (Q4_0, Q8_0, Q4_K; G = 1,
     // 2, 4; sbw 2, 4), and the same classes of the fused gate/up (sbw 4)
     hipFunction_t mmqt[RQ_NUM_FMTS][3][2] = {};
@@ -262,6 +263,13 @@ struct rq_ctx {
     hipFunction_t mmqdw[RQ_NUM_FMTS][3] = {};
     hipFunction_t mmqgluw[RQ_NUM_FMTS][4] = {};
     hipFunction_t mmq_repack[RQ_NUM_FMTS] = {};
+    // Column kernels (rq_cols.hip) by format (RQ_NUM_FMTS: mixed Q4_K /
+    // Q6_K), layout (0: dot4, 1: MFMA), tiles per workgroup (1, 2, 4) and
+    // column groups, null where there is none; the fused gate/up ones by
+    // column groups.
+    hipModule_t cols_mod = nullptr;
+    hipFunction_t cols[RQ_NUM_FMTS + 1][2][3][RQ_COLS_MAX_GROUPS] = {};
+    hipFunction_t colsglu[RQ_NUM_FMTS][2] = {};
     // The f16 GEMM route of batched rq_matmul* (rq_set_gemm_min_m): f16
     // dequantization from either layout, f32 -> f16, rocBLAS (created by the
     // first such call or rq_reserve_f16, with a fixed workspace), and the
@@ -663,14 +671,13 @@ bool mmq_has_t(int fmt, int S2) { return fmt != RQ_FMT_MIX_K && (S2 + 3) / 4 <= 
 // Q6_K runs the 16-column kernels for up to 16 columns only: holding its
 // weights for a second group makes them spill.
 int mmqt_max_cols(int fmt) { return fmt == RQ_FMT_Q6_K ? 16 : 64; }
-// Q6_K takes up to 64 in its 8-column classes (8 x 6, 8 x 8 add each group's
-// k-parts as it ends, so LDS holds one group's partial sums next to 8 staged
-// columns of a 14336-wide row).
+// (Q6_K, and so its mix with Q4_K, comes here with at most 16 columns:
+// use_cols.)
 int mmq_max_cols(int fmt, int S2) {
-    return mmq_np(fmt, S2) > 1 ? 8 : (mmq_has_t(fmt, S2) || fmt == RQ_FMT_Q6_K) && fmt != RQ_FMT_MIX_K ? 64 : 32;
+    return mmq_np(fmt, S2) > 1 ? 8 : fmt == RQ_FMT_Q6_K || fmt == RQ_FMT_MIX_K ? 16 : mmq_has_t(fmt, S2) ? 64 : 32;
 }
 // Table index of an 8 x g class.
-int mmqg_index(int g) { return g == 2 ? 0 : g == 4 ? 1 : g == 6 ? 2 : 3; }
+int mmqg_index(int g) { return g == 2 ? 0 : 1; }
 // Group-count index of a 16-column class (g = 1, 2, 4).
 int mmqt_g_index(int g) { return g == 1 ? 0 : g == 2 ? 1 : 2; }
 // Super-blocks per wave of a 16-column launch: 4 for Q4_K; 2 for Q4_0 and
@@ -741,8 +748,7 @@ void mmq_layout(int fmt, int S2, bool dots, MmqPlan& L) {
     L.kxp = S2 * 256 + 64;  // 64 B of skew: columns start on different LDS banks
     L.pl_off = L.mp * L.kxp;
     L.part_off = L.pl_off + (mmq_planes(fmt) + (dots ? 1 : 0)) * L.mp * RQ_MMQ_NBP(S2) * 4;
-    // Partial sums of every group, or (g > 4) of one group at a time.
-    L.lds = L.part_off + (dots ? 0 : L.ks * L.tr * 64 * (L.mp == 8 ? 2 : 1) * (L.g > 4 ? 1 : L.g) * 4);
+    L.lds = L.part_off + (dots ? 0 : L.ks * L.tr * 64 * (L.mp == 8 ? 2 : 1) * L.g * 4);  // every group's partial sums
 }
 
 // A Q6_K vocabulary head (>= 16384 rows of 9 to 16 super-blocks) at one
@@ -870,7 +876,7 @@ MmqPlan mmq_cols(int fmt, int S2, int nc, bool allow16 = true) {
         return L;
     }
     L.mp = nc <= 1 ? 1 : nc <= 4 ? 4 : 8;
-    L.g = nc <= 8 ? 1 : nc <= 16 ? 2 : nc <= 32 || fmt != RQ_FMT_Q6_K ? 4 : nc <= 48 ? 6 : 8;
+    L.g = nc <= 8 ? 1 : nc <= 16 ? 2 : 4;
     return L;
 }
 
@@ -969,6 +975,221 @@ rq_status mmq_launch(rq_ctx* ctx, const int8_t* xq, const uint16_t* xd, const fl
         g0 += nc;
     }
     return RQ_OK;
+}
+
+// ---------------------------------------------------------------------------
+// Column kernels (rq_cols.hip).
+
+// LDS of a workgroup of rt tiles and cg column groups over rows of S
+// super-blocks: the staged chunks of eight super-blocks (dot4 layout; Q6_K
+// also their f16 d), the waves' staged activations and the columns' scales; at the end the eight waves' sums.
+int cols_lds_bytes(int fmt, bool mfma, int rt, int cg, int S) {
+    const int f = fmt == RQ_FMT_MIX_K ? RQ_FMT_Q6_K : fmt;
+    const int stage = mfma ? 0 : 16 * rt * 8 * (rq_chunks(f) * 16 + (f == RQ_FMT_Q6_K ? 2 : 0));
+    const int x = RQ_COLS_PARTS * cg * 16 * RQ_COLS_XCOL + 16 * cg * (16 * S + 8);
+    return std::max(stage + x, RQ_COLS_PARTS * rt * cg * 1024);
+}
+
+// Most tiles per workgroup there is a kernel for (more would spill).
+int cols_max_rt(bool mfma, int cg) { return cg <= 2 ? (mfma ? 2 : 4) : cg == 3 ? 2 : 1; }
+
+// Launches of m columns over `tiles` 16-row tiles: rt tiles per workgroup and
+// cg column groups per launch, rt = 0 where nothing fits the LDS.
+//   rt: tiles of a workgroup share its reads and conversion of the
+//       activations, but a launch wants a workgroup for every CU. Q4_K, dot4
+//       layout at 16 columns, 1 / 2 / 4 tiles: 4096 x 4096 (256 tiles) 7.4 /
+//       9.0 / 13.6 us, 14336 x 4096 (896 tiles) 17.0 / 16.5 / 13.9 us.
+//   cg: 64 columns in one launch hold one tile per workgroup (15.3 us for
+//       4096 x 4096), so weights that want two or more go as two launches of
+//       32 (14336 x 4096: 56.3 us in one launch, 18.7 in each of two).
+struct ColsPlan {
+    int rt = 0, cg = 0;
+    int64_t launches = 0;
+};
+ColsPlan cols_plan(const rq_ctx* ctx, int fmt, bool mfma, int64_t tiles, int S, int64_t m) {
+    ColsPlan p;
+    const bool many = tiles > ctx->cus * 3 / 2;
+    for (int max_cg = many ? 3 : RQ_COLS_MAX_GROUPS; max_cg >= 1; max_cg--) {
+        const int64_t per = RQ_COLS_GROUP * max_cg;
+        p.launches = (m + per - 1) / per;
+        p.cg = (int)(((m + p.launches - 1) / p.launches + RQ_COLS_GROUP - 1) / RQ_COLS_GROUP);
+        int rt = std::min(cols_max_rt(mfma, p.cg), tiles >= 3 * ctx->cus ? 4 : many ? 2 : 1);
+        for (; rt >= 1; rt /= 2)
+            if (cols_lds_bytes(fmt, mfma, rt, p.cg, S) <= ctx->lds_wide) {
+                p.rt = rt;
+                return p;
+            }
+    }
+    return p;
+}
+
+// The fused gate/up launches (dot4 layout): two tiles of each weight per
+// workgroup and at most two column groups; 0 where that does not fit the LDS.
+int cols_glu_groups(const rq_ctx* ctx, int fmt, int S) {
+    int cg = 2;
+    while (cg > 0 && cols_lds_bytes(fmt, false, 4, cg, S) > ctx->lds_wide) cg--;
+    return cg;
+}
+
+// Whether m columns of w run the column kernels.
+//   dot4 layout: past the 8 columns of one dot4 launch, each further 8 of
+//     which would read the weights again (us, dot4 / column kernels at 16 and
+//     64 columns: Q4_K 4096 x 4096 17.5 / 7.3 and 69.7 / 15.6, 14336 x 4096
+//     36.7 / 13.7 and 144 / 37.5; Q8_0 11008 x 4096 30.5 / 17.4 and 120 / 44;
+//     Q6_K 4096 x 14336 65 / 20 and 180 / 43, 128256 x 4096 227 / 144 and 894
+//     / 390); rows of more than 32 super-blocks, one to a tile there, from 7
+//     (Q6_K 4096 x 14336 at 6 / 8: 20.1 / 32.0 against 20.1). At 8 columns
+//     4096-wide weights are mixed (Q4_K 4096 x 4096 9.3 / 7.3, Q6_K 14336 x
+//     4096 18.7 / 20.4).
+//   MFMA layout: Q6_K past 16 columns (1024 x 4096 at 32 / 64: 14.9 / 31.4
+//     us in its 8-column classes, 9.2 / 14.9 here; 14336 x 4096 at 32 28.0 /
+//     26.3), wide rows, which its 16-column class cannot stage, past 8 (4096
+//     x 14336 at 16 / 32 / 64: 22.0 / 37.9 / 72.9 -> 17.9 / 25.3 / 42.9 us;
+//     past 64 super-blocks every type, whose classes stop at 8 columns there);
+//     the other types past 16 columns up to 512 tiles (Q4_K 4096 x 4096 at 32
+//     / 48 / 64: 10.9 / 17.8 / 19.0 -> 9.3 / 11.9 / 15.0 us; Q4_0 11.1 / 17.7
+//     / 19.0 -> 9.0 / 11.3 / 14.1), above which their classes read the
+//     activations for four tiles at once (Q4_K 14336 x 4096 at 32: 18.9
+//     against 22.4 us).
+// By the weight and m alone, so that a weight's result does not depend on
+// the weights beside it.
+bool use_cols(const rq_ctx* ctx, const rq_weight* w, int64_t m) {
+    const int S = (int)((w->cols + 255) / 256);
+    const bool mfma = use_mmq(w, m);
+    bool use;
+    if (!mfma)
+        use = m >= (S > 32 ? 7 : 9);
+    else if (S > 64 || (S > 32 && w->fmt == RQ_FMT_Q6_K))
+        use = m > 8;
+    else
+        use = m > 16 && (w->fmt == RQ_FMT_Q6_K || w->tiles <= 512);
+    return use && cols_plan(ctx, w->fmt, mfma, 1, S, m).rt > 0;
+}
+
+int log2_of(int v) {
+    int l = 0;
+    while ((1 << l) < v) l++;
+    return l;
+}
+
+void cols_params(RqColsParams& p, const rq_weight* w, bool mfma, const int8_t* xq, const uint16_t* xd, int64_t nc) {
+    memset(&p, 0, sizeof p);
+    p.xq = xq;
+    p.xd = xd;
+    p.m = (int32_t)nc;
+    p.k = (int32_t)w->cols;
+    p.S = (int32_t)((w->cols + 255) / 256);
+    p.lr = mfma ? 0 : log2_of(w->tiled.R);
+    p.S2 = w->S2;
+}
+
+RqColsTarget cols_target(const rq_weight* w, bool mfma) {
+    RqColsTarget t;
+    memset(&t, 0, sizeof t);
+    t.a = mfma ? w->code : w->tiled.main;
+    t.b = mfma ? w->hdr : w->tiled.tail;
+    t.n = (int32_t)w->rows;
+    t.tiles = (int32_t)((w->rows + 15) / 16);
+    t.fmt = w->fmt;
+    return t;
+}
+
+// Matvec launches over `count` weights of one width and layout, Q8_1 columns
+// in near-equal launches of at most 64.
+rq_status cols_launch(rq_ctx* ctx, const int8_t* xq, const uint16_t* xd, int64_t m, const rq_weight* const* ws,
+                      float* const* outs, int count) {
+    const bool mfma = use_mmq(ws[0], m);
+    int fmt = ws[0]->fmt;
+    int64_t tiles = 0;
+    for (int i = 0; i < count; i++) {
+        if (ws[i]->fmt != fmt) fmt = RQ_FMT_MIX_K;
+        tiles += (ws[i]->rows + 15) / 16;
+    }
+    const int64_t k = ws[0]->cols;
+    const int S = (int)((k + 255) / 256);
+    const ColsPlan plan = cols_plan(ctx, fmt, mfma, tiles, S, m);
+    if (plan.rt == 0) return fail(RQ_ERR_SHAPE, "matvec: %lld columns too wide to stage", (long long)k);
+    const int rt = plan.rt;
+    for (int64_t gi = 0, g0 = 0; gi < plan.launches; gi++) {
+        const int64_t nc = m / plan.launches + (gi < m % plan.launches ? 1 : 0);
+        const int cg = (int)((nc + RQ_COLS_GROUP - 1) / RQ_COLS_GROUP);
+        RqColsParams p;
+        cols_params(p, ws[0], mfma, xq + g0 * k, xd + g0 * (k / 32), nc);
+        p.count = count;
+        int64_t wgs = 0;
+        int o = 0;
+        for (int pass = 0; pass < 2; pass++)  // Q6_K targets first: their workgroups carry more work
+            for (int i = 0; i < count; i++) {
+                if ((ws[i]->fmt == RQ_FMT_Q6_K) != (pass == 0)) continue;
+                p.t[o] = cols_target(ws[i], mfma);
+                p.t[o].out = outs[i] + g0 * ws[i]->rows;
+                p.t[o].wg_start = (int32_t)wgs;
+                wgs += (p.t[o].tiles + rt - 1) / rt;
+                o++;
+            }
+        rq_status st = launch(ctx, ctx->cols[mmq_fi(fmt)][mfma ? 1 : 0][rt >> 1][cg - 1], "rq_cols", (uint64_t)wgs, &p,
+                              (unsigned)cols_lds_bytes(fmt, mfma, rt, cg, S), RQ_COLS_THREADS);
+        if (st != RQ_OK) return st;
+        g0 += nc;
+    }
+    return RQ_OK;
+}
+
+// Gate and up of one type and shape in the dot4 layout through rq_colsglu_*:
+// from 6 columns (Q4_K 14336 x 4096 at 6: 34.0 us in rq_glu_*, 32.1 here; at
+// 16 two launches there).
+bool cols_glu_ok(const rq_ctx* ctx, const rq_weight* gate, const rq_weight* up, int64_t m) {
+    return m >= 6 && glu_fusable(gate, up, m) &&
+           cols_glu_groups(ctx, gate->fmt, (int)((gate->cols + 255) / 256)) > 0;
+}
+
+// h = act(x . gate) * (x . up) of Q8_1 columns into hf (may be null) and its
+// Q8_1 (hq, hd, hs; may be null).
+rq_status cols_glu_launch(rq_ctx* ctx, const int8_t* xq, const uint16_t* xd, int64_t m, const rq_weight* gate,
+                          const rq_weight* up, int act, float* hf, int8_t* hq, uint16_t* hd, uint16_t* hs) {
+    const int64_t k = gate->cols, n = gate->rows;
+    const int64_t max_cols = RQ_COLS_GROUP * cols_glu_groups(ctx, gate->fmt, (int)((k + 255) / 256));
+    const int64_t ngroups = (m + max_cols - 1) / max_cols;
+    for (int64_t gi = 0, g0 = 0; gi < ngroups; gi++) {
+        const int64_t nc = m / ngroups + (gi < m % ngroups ? 1 : 0);
+        const int cg = (int)((nc + RQ_COLS_GROUP - 1) / RQ_COLS_GROUP);
+        RqColsParams p;
+        cols_params(p, gate, false, xq + g0 * k, xd + g0 * (k / 32), nc);
+        p.t[0] = cols_target(gate, false);
+        p.t[1] = cols_target(up, false);
+        p.count = 2;
+        p.act = act;
+        p.hf = hf ? hf + g0 * n : nullptr;
+        if (hq) {
+            p.hq = hq + g0 * n;
+            p.hd = hd + g0 * n / 32;
+            p.hs = hs + g0 * n / 32;
+        }
+        rq_status st = launch(ctx, ctx->colsglu[gate->fmt][cg - 1], "rq_colsglu", (uint64_t)(n / 32), &p,
+                              (unsigned)cols_lds_bytes(gate->fmt, false, 4, cg, p.S), RQ_COLS_THREADS);
+        if (st != RQ_OK) return st;
+        g0 += nc;
+    }
+    return RQ_OK;
+}
+
+// One matvec group (one width and family) over Q8_1 activations: the weights
+// that run the column kernels in one launch, the others in another.
+rq_status matvec_dispatch(rq_ctx* ctx, const int8_t* xq, const uint16_t* xd, int64_t m, const rq_weight* const* ws,
+                          float* const* outs, int count) {
+    const rq_weight* w[2][RQ_MV_TARGETS];
+    float* o[2][RQ_MV_TARGETS];
+    int n[2] = {0, 0};
+    for (int i = 0; i < count; i++) {
+        const int c = use_cols(ctx, ws[i], m) ? 1 : 0;
+        w[c][n[c]] = ws[i];
+        o[c][n[c]++] = outs[i];
+    }
+    rq_status st = RQ_OK;
+    if (n[1] > 0) st = cols_launch(ctx, xq, xd, m, w[1], o[1], n[1]);
+    if (st != RQ_OK || n[0] == 0) return st;
+    if (use_mmq(w[0][0], m)) return mmq_launch(ctx, xq, xd, nullptr, m, w[0], (void* const*)o[0], n[0], false);
+    return matvec_launch(ctx, xq, xd, nullptr, m, w[0], o[0], n[0]);
 }
 
 // Fused gate/up + activation over the MFMA layout (rq_mmqglu_*): gate and up
@@ -1198,6 +1419,7 @@ extern "C" rq_status rq_open(int device, rq_ctx** out) {
         if (ctx->up_stream) (void)hipStreamDestroy(ctx->up_stream);
         if (ctx->mod) (void)hipModuleUnload(ctx->mod);
         if (ctx->mmq_mod) (void)hipModuleUnload(ctx->mmq_mod);
+        if (ctx->cols_mod) (void)hipModuleUnload(ctx->cols_mod);
         delete ctx;
         return st;
     };
@@ -1218,6 +1440,7 @@ extern "C" rq_status rq_open(int device, rq_ctx** out) {
         return bail(fail(RQ_ERR_UNSUPPORTED, "rq_open: device %d is %s; librq is built for gfx950 only", device, ctx->arch));
     if ((e = hipModuleLoadData(&ctx->mod, rq_kernels_blob)) != hipSuccess) return bail(hip_fail("hipModuleLoadData", e));
     if ((e = hipModuleLoadData(&ctx->mmq_mod, rq_mmq_blob)) != hipSuccess) return bail(hip_fail("hipModuleLoadData", e));
+    if ((e = hipModuleLoadData(&ctx->cols_mod, rq_cols_blob)) != hipSuccess) return bail(hip_fail("hipModuleLoadData", e));
     auto getm = [&](hipModule_t mod, hipFunction_t* f, const char* name) -> rq_status {
         hipError_t ge = hipModuleGetFunction(f, mod, name);
         if (ge != hipSuccess)
@@ -1284,8 +1507,7 @@ extern "C" rq_status rq_open(int device, rq_ctx** out) {
             if (kMmqSbw[si] > mmq_sbw_max(f)) continue;
             snprintf(name, sizeof name, "rq_mmqf_%s_%d", kFmtSuffix[f], kMmqSbw[si]);
             st = getm(ctx->mmq_mod, &ctx->mmqf[f][si], name);
-            for (int gi = 0; gi < 4 && st == RQ_OK; gi++) {
-                if (gi >= 2 && (f != RQ_FMT_Q6_K || kMmqSbw[si] != 4)) continue;  // 8 x 6, 8 x 8: Q6_K only
+            for (int gi = 0; gi < (f == RQ_FMT_Q6_K ? 1 : 2) && st == RQ_OK; gi++) {
                 snprintf(name, sizeof name, "rq_mmq_%s_8x%d_%d", kFmtSuffix[f], 2 * (gi + 1), kMmqSbw[si]);
                 st = getm(ctx->mmq_mod, &ctx->mmqg[f][gi][si], name);
             }
@@ -1341,13 +1563,24 @@ extern "C" rq_status rq_open(int device, rq_ctx** out) {
         const int fi = RQ_NUM_FMTS;
         snprintf(name, sizeof name, "rq_mmqf_q4_k_q6_k_%d", kMmqSbw[si]);
         st = getm(ctx->mmq_mod, &ctx->mmqf[fi][si], name);
-        for (int gi = 0; gi < 2 && st == RQ_OK; gi++) {
-            snprintf(name, sizeof name, "rq_mmq_q4_k_q6_k_8x%d_%d", 2 << gi, kMmqSbw[si]);
-            st = getm(ctx->mmq_mod, &ctx->mmqg[fi][gi][si], name);
-        }
+        snprintf(name, sizeof name, "rq_mmq_q4_k_q6_k_8x2_%d", kMmqSbw[si]);
+        if (st == RQ_OK) st = getm(ctx->mmq_mod, &ctx->mmqg[fi][0][si], name);
         for (int mi = 0; mi < 3 && st == RQ_OK; mi++) {
             snprintf(name, sizeof name, "rq_mmq_q4_k_q6_k_%d_%d", kMmqMp[mi], kMmqSbw[si]);
             st = getm(ctx->mmq_mod, &ctx->mmq[fi][mi][si], name);
+        }
+    }
+    for (int f = 0; f <= RQ_NUM_FMTS && st == RQ_OK; f++) {
+        const char* fs = f == RQ_NUM_FMTS ? "q4_k_q6_k" : kFmtSuffix[f];
+        for (int l = 0; l < 2 && st == RQ_OK; l++)
+            for (int cg = 1; cg <= RQ_COLS_MAX_GROUPS && st == RQ_OK; cg++)
+                for (int rt = 1; rt <= cols_max_rt(l == 1, cg) && st == RQ_OK; rt *= 2) {
+                    snprintf(name, sizeof name, "rq_cols_%s_%c_%dx%d", fs, "dm"[l], rt, cg);
+                    st = getm(ctx->cols_mod, &ctx->cols[f][l][rt >> 1][cg - 1], name);
+                }
+        for (int cg = 1; cg <= 2 && f < RQ_NUM_FMTS && st == RQ_OK; cg++) {
+            snprintf(name, sizeof name, "rq_colsglu_%s_%d", fs, cg);
+            st = getm(ctx->cols_mod, &ctx->colsglu[f][cg - 1], name);
         }
     }
     if (st != RQ_OK) return bail(st);
@@ -1432,6 +1665,7 @@ extern "C" rq_status rq_close(rq_ctx* ctx) {
         if (ctx->up_stream) (void)hipStreamDestroy(ctx->up_stream);
         if (ctx->mod) (void)hipModuleUnload(ctx->mod);
         if (ctx->mmq_mod) (void)hipModuleUnload(ctx->mmq_mod);
+        if (ctx->cols_mod) (void)hipModuleUnload(ctx->cols_mod);
     }
     if (st != RQ_OK)  // the device could not be bound: detach the weights all the same
         for (rq_weight* w : ctx->live) w->ctx = nullptr;
@@ -1806,8 +2040,7 @@ extern "C" rq_status rq_matvec_many(rq_ctx* ctx, const rq_q8_1* xq, int64_t m, c
         if ((st = check_len("matmul out", out_lens[i], m * ws[i]->rows)) != RQ_OK) return st;
     if (m == 0) return RQ_OK;
     if ((st = bind(ctx)) != RQ_OK) return st;
-    if (use_mmq(ws[0], m)) return mmq_launch(ctx, xq->qs, xq->d, nullptr, m, ws, (void* const*)outs, count, false);
-    return matvec_launch(ctx, xq->qs, xq->d, nullptr, m, ws, outs, count);
+    return matvec_dispatch(ctx, xq->qs, xq->d, m, ws, outs, count);
 }
 
 extern "C" rq_status rq_matvec(rq_ctx* ctx, const rq_q8_1* xq, int64_t m, const rq_weight* w, float* out,
@@ -2148,12 +2381,12 @@ rq_status matmul_many_run(rq_ctx* ctx, const float* x, int64_t x_len, int64_t m,
             if (!ok) break;
             g++;
         }
-        if (use_mmq(ws[i], m))
-            st = fused ? mmq_launch(ctx, nullptr, nullptr, x, m, ws + i, (void* const*)(outs + i), g, false)
-                       : mmq_launch(ctx, sc.q, sc.d, nullptr, m, ws + i, (void* const*)(outs + i), g, false);
+        if (!fused)
+            st = matvec_dispatch(ctx, sc.q, sc.d, m, ws + i, outs + i, g);
+        else if (use_mmq(ws[i], m))
+            st = mmq_launch(ctx, nullptr, nullptr, x, m, ws + i, (void* const*)(outs + i), g, false);
         else
-            st = fused ? matvec_launch(ctx, nullptr, nullptr, x, m, ws + i, outs + i, g)
-                       : matvec_launch(ctx, sc.q, sc.d, nullptr, m, ws + i, outs + i, g);
+            st = matvec_launch(ctx, nullptr, nullptr, x, m, ws + i, outs + i, g);
         if (st != RQ_OK) return st;
         i += g;
     }
@@ -2225,13 +2458,6 @@ namespace {
 
 const char* act_name(int act) { return act == RQ_ACT_GELU_TANH ? "gelu_mul" : "silu_mul"; }
 
-// One matvec group (same type and family) over Q8_1 activations.
-rq_status matvec_dispatch(rq_ctx* ctx, const int8_t* xq, const uint16_t* xd, int64_t m, const rq_weight* const* ws,
-                          float* const* outs, int count) {
-    if (use_mmq(ws[0], m)) return mmq_launch(ctx, xq, xd, nullptr, m, ws, (void* const*)outs, count, false);
-    return matvec_launch(ctx, xq, xd, nullptr, m, ws, outs, count);
-}
-
 // Shared checks of rq_glu_matmul / rq_gated_ffn: gate and up of one shape, x
 // of m rows of their width.
 rq_status check_glu_shape(const rq_ctx* ctx, const char* what, int64_t m, const rq_weight* gate, const rq_weight* up,
@@ -2287,6 +2513,20 @@ rq_status glu_run(rq_ctx* ctx, const float* x, const rq_q8_1* xq, int64_t m, con
         const int64_t lens[2] = {m * n, m * n};
         if ((st = rq_matmul_many(ctx, x, m * k, m, ws, outs, lens, 2)) != RQ_OK) return st;
         return act_mul_launch(ctx, act, hf, ub, m * n, hq, hd, hs);
+    }
+    if (cols_glu_ok(ctx, gate, up, m)) {
+        const int8_t* q = xq ? xq->qs : nullptr;
+        const uint16_t* d = xq ? xq->d : nullptr;
+        if (!xq) {
+            if ((st = ensure_scratch(ctx, m * k)) != RQ_OK) return st;
+            RqQuantParams qp{x, ctx->sq, ctx->sd, ctx->ss, m * k / 32};
+            if ((st = launch(ctx, ctx->quant, "rq_quantize_q8_1",
+                             (uint64_t)((qp.nblocks * 8 + RQ_THREADS - 1) / RQ_THREADS), &qp)) != RQ_OK)
+                return st;
+            q = ctx->sq;
+            d = ctx->sd;
+        }
+        return cols_glu_launch(ctx, q, d, m, gate, up, act, hf, hq, hd, hs);
     }
     if (glu_mmq_ok(gate, up, m)) {
         if (xq) return mmq_glu_launch(ctx, xq->qs, xq->d, nullptr, m, gate, up, act, hf, hq, hd, hs);
@@ -2461,7 +2701,7 @@ rq_status gated_ffn_run(rq_ctx* ctx, const char* what, const float* x, int64_t x
                     (long long)n);
     if ((st = check_len("gated_ffn gate", gate_len, m * n)) != RQ_OK) return st;
     if ((st = check_len("matmul out", out_len, m * down->rows)) != RQ_OK) return st;
-    if (!glu_fusable(gate, up, m) && !glu_mmq_ok(gate, up, m) &&
+    if (!glu_fusable(gate, up, m) && !glu_mmq_ok(gate, up, m) && !cols_glu_ok(ctx, gate, up, m) &&
         (st = check_len("gated_ffn up", up_len, m * n)) != RQ_OK)
         return st;
     // The f16 GEMM route (f32 x) writes up's product to up_buf when given.

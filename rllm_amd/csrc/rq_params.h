@@ -213,6 +213,49 @@ struct RqMmqParams {
     int32_t np;  // passes per wave over the row (rows wider than ks * sbw super-blocks; 0 or 1: one)
 };
 
+// ---------------------------------------------------------------------------
+// The column kernels (rq_cols_* / rq_colsglu_* in rq_cols.hip): 4 to 64 Q8_1
+// columns against either weight layout.
+
+// Threads per workgroup: eight waves, wave w taking the super-blocks s of a
+// row with s % 8 == w.
+#define RQ_COLS_THREADS 512
+#define RQ_COLS_PARTS (RQ_COLS_THREADS / 64)
+// Columns per group (the N of an MFMA) and most groups per launch.
+#define RQ_COLS_GROUP 16
+#define RQ_COLS_MAX_GROUPS 4
+
+// LDS bytes of a staged column's half super-block (16 of skew).
+#define RQ_COLS_XCOL 144
+
+struct RqColsTarget {
+    const uint8_t* a;   // dot4 layout: chunk plane; MFMA layout: code plane
+    const uint8_t* b;   // dot4 layout: Q6_K tail plane; MFMA layout: header plane
+    float* out;         // out[j * n + r]
+    int32_t n;          // rows
+    int32_t wg_start;   // first workgroup of this target
+    int32_t fmt;        // RQ_FMT_* (read by the mixed Q4_K / Q6_K kernels)
+    int32_t tiles;      // 16-row tiles
+};
+
+struct RqColsParams {
+    RqColsTarget t[RQ_MV_TARGETS];
+    const int8_t* xq;    // Q8_1 codes, column j at xq + j * k
+    const uint16_t* xd;  // Q8_1 f16 scales, column j at xd + j * k / 32
+    int32_t count;
+    int32_t m;           // columns of this launch
+    int32_t k;
+    int32_t S;           // super-blocks per row, ceil(k / 256)
+    int32_t lr;          // dot4 layout: log2 of the rows per tile
+    int32_t S2;          // MFMA layout: stored super-blocks per row
+    int32_t act;         // rq_colsglu_*: RQ_ACT_*
+    int32_t pad;
+    float* hf;           // rq_colsglu_*: the product h (f32, may be null) and its Q8_1 (may be null)
+    int8_t* hq;
+    uint16_t* hd;
+    uint16_t* hs;
+};
+
 struct RqMmqRepackParams {
     const uint8_t* raw;  // GGUF bytes of rows [row0, row0 + rows)
     uint8_t* code;

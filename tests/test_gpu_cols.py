@@ -1,0 +1,117 @@
+"""The column kernels (rq_cols_*, rq_colsglu_*): matvecs over more than 8
+Q8_1 columns, and the dot4 layout's fused gate/up from 6, against the integer
+oracle at the edges of their tiles, column groups and rows."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import make_weight, q8_1_to_device, upload
+from rllm_amd.backend import Activation
+
+pytestmark = pytest.mark.gpu
+
+TYPES = {"Q4_0": 2, "Q8_0": 8, "Q4_K": 12, "Q6_K": 14}
+
+# f32 sums over exact products: a row of S super-blocks passes at most 4 + 1
+# roundings per half super-block, 2 ceil(S / 8) partial sums and 3 levels of
+# eight parts, each 2^-24 of a partial sum. Partial sums of N(0, 1) terms stay
+# within about the row's norm, so 1e-5 of the largest output (170 roundings,
+# all one way) is out of reach for the widths here.
+TOL = 1e-5
+
+
+def _q8(orc, seed, m, k):
+    return orc.quantize_q8_1(orc.normal(seed, m * k, 0.0, 1.0), m, k)
+
+
+@pytest.mark.parametrize("tname", list(TYPES))
+@pytest.mark.parametrize("n,k", [(1, 256), (16, 512), (17, 2048), (63, 2304), (96, 4096), (33, 13824), (37, 16896),
+                                 (40, 32), (24, 160), (50, 2080)])
+@pytest.mark.parametrize("m", [9, 16, 17, 43, 64, 70])
+def test_cols_matvec(gpu, orc, tname, n, k, m):
+    """Both layouts against the oracle, and bit-identical to each other
+    wherever both run the column kernels (m > 16, or wide rows): the order of
+    the sums depends on the width alone."""
+    t = TYPES[tname]
+    if t in (12, 14) and k % 256:
+        pytest.skip("K-quants need k % 256 == 0")
+    w = make_weight(orc, t, n, k, 40 + n, "random")
+    qs, d, s = _q8(orc, 41 + k + m, m, k)
+    want = orc.matvec_q8_1(t, w, n, k, qs, d, m)
+    got = {}
+    for fam in ("dot4", "mfma"):
+        gpu.set_kernels(fam)
+        wg = upload(gpu, t, w, n, k)
+        gpu.set_kernels("auto")
+        out = gpu.alloc(m * n + 8)
+        out.fill_(float("nan"))
+        gpu.matvec(q8_1_to_device(gpu, qs, d, s), wg, out, m)
+        got[fam] = gpu.to_host(out)
+        assert np.isnan(got[fam][m * n:]).all(), "wrote past the output"
+        orc.assert_close(f"{tname} {n}x{k} m={m} {fam}", want, got[fam][:m * n], TOL if m > 16 or fam == "dot4" else 1e-3)
+    if m > 16:
+        assert np.array_equal(got["dot4"][:m * n].view(np.uint32), got["mfma"][:m * n].view(np.uint32))
+
+
+@pytest.mark.parametrize("tname", list(TYPES))
+def test_cols_do_not_depend_on_the_count(gpu, orc, tname):
+    """The first columns of a 70-column call (two launches) as calls of 9 and
+    33, and of rows enough for two and four tiles per workgroup."""
+    t, k = TYPES[tname], 1024
+    for n in (40, 16 * 400, 16 * 800):
+        w = orc.random_weight(50, t, n, k)
+        wg = upload(gpu, t, w, n, k)
+        qs, d, s = _q8(orc, 51, 70, k)
+        outs = {}
+        for m in (70, 33, 9):
+            out = gpu.alloc(m * n)
+            xq = q8_1_to_device(gpu, qs[:m * k], d[:m * k // 32], s[:m * k // 32])
+            gpu.matvec(xq, wg, out, m)
+            outs[m] = gpu.to_host(out, m * n).view(np.uint32)
+        for m in (33, 9):
+            assert np.array_equal(outs[m], outs[70][:m * n]), f"n={n} m={m}"
+        rows = np.r_[0:20, n - 20:n]
+        want = orc.matvec_q8_1(t, w, n, k, qs[:9 * k], d[:9 * k // 32], 9).reshape(9, n)
+        orc.assert_close(f"{tname} {n}x{k}", want[:, rows].reshape(-1),
+                         outs[9].view(np.float32).reshape(9, n)[:, rows].reshape(-1), TOL)
+
+
+@pytest.mark.parametrize("family", ["dot4", "mfma"])
+@pytest.mark.parametrize("k", [4096, 13824])
+def test_cols_mixed_launch(gpu, orc, family, k):
+    """Q4_K and Q6_K weights together are bit-identical to their own calls,
+    whichever of them run the column kernels (MFMA: Q6_K does at 20 columns,
+    a Q4_K weight of more than 512 tiles does not)."""
+    m = 20
+    spec = [(12, 48), (14, 33), (12, 8208 if k == 4096 else 17)]
+    ws = [orc.random_weight(60 + i, t, n, k) for i, (t, n) in enumerate(spec)]
+    gpu.set_kernels(family)
+    wgs = [upload(gpu, t, w, n, k) for (t, n), w in zip(spec, ws)]
+    gpu.set_kernels("auto")
+    x = gpu.from_host(orc.normal(61, m * k, 0.0, 1.0))
+    outs = [gpu.alloc(m * n) for _, n in spec]
+    gpu.matmul_many(x, wgs, outs, m)
+    for (t, n), wg, out in zip(spec, wgs, outs):
+        own = gpu.alloc(m * n)
+        gpu.matmul(x, wg, own, m)
+        assert torch.equal(own.view(torch.int32), out.view(torch.int32)), f"type {t} rows {n}"
+
+
+@pytest.mark.parametrize("tname", list(TYPES))
+@pytest.mark.parametrize("f,d", [(32, 512), (96, 4096), (64, 5120)])
+@pytest.mark.parametrize("m", [5, 6, 16, 17, 33, 50])
+def test_cols_gated_ffn(gpu, orc, tname, f, d, m):
+    """The dot4 layout's fused front half: h within 1e-3 of the integer path
+    (the activation's expf), the down projection on exactly h's Q8_1."""
+    t = TYPES[tname]
+    gw, uw = orc.random_weight(70, t, f, d), orc.random_weight(71, t, f, d)
+    g, u = upload(gpu, t, gw, f, d), upload(gpu, t, uw, f, d)
+    qs, dq, s = _q8(orc, 73 + m, m, d)
+    h = gpu.alloc(m * f)
+    out = gpu.alloc(m * 256)
+    down = upload(gpu, 8, orc.random_weight(74, 8, 256, f), 256, f)
+    gpu.gated_ffn_q8_1(q8_1_to_device(gpu, qs, dq, s), g, u, down, Activation.SILU, out, h, gpu.alloc(m * f), m)
+    orc.assert_close(f"h {tname} {f}x{d} m={m}", orc.glu_q8_1(t, gw, uw, f, d, qs, dq, m, 0), gpu.to_host(h, m * f), 1e-3)
+    want = gpu.alloc(m * 256)
+    gpu.matvec(gpu.quantize_q8_1(h, m, f), down, want, m)
+    assert torch.equal(out.view(torch.int32), want.view(torch.int32))
