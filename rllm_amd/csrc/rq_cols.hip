@@ -1,7 +1,8 @@
 // Matvecs over more than 8 activation columns (rq_cols_*, either weight
 // layout, rq_params.h) and the fused gate/up front half of a gated FFN from 6
-// (rq_colsglu_*, the dot4 layout). Which calls come here, and both sides'
-// times: use_cols in rq_host.cpp.
+// (rq_colsglu_*, the dot4 layout); on the same weight sources the f16 GEMM
+// route's kernels for short prompts (rq_gemm_*, at the end). Which calls come
+// here, and both sides' times: use_cols and gemm_fused in rq_host.cpp.
 //
 // What bounds them. Every weight is read once, so a launch cannot be faster
 // than its bytes; up to about 16 columns that is the bound. The work beside
@@ -156,7 +157,7 @@ struct HalfW {
     u32 sc, mn;    // Q4_K: the four blocks' scales and mins (row n)
     u32 sc6[2];    // Q6_K: the eight sub-block scales (row n)
     u32 dd;        // Q4_K: f16 d, dmin of row n
-    u32 d[4][2];   // rows 4 g + e: d (Q4_K / Q6_K: [e][0] low half) or the four blocks' d (Q4_0 / Q8_0)
+    u32 d[4][2];   // rows 4 g + e (OWN: [0] only, row n): d (Q4_K / Q6_K: [e][0] low half) or the four blocks' d (Q4_0 / Q8_0)
 };
 
 __device__ __forceinline__ void q4k_half(const int4& h, int hb, u32& sc, u32& mn) {
@@ -167,6 +168,8 @@ __device__ __forceinline__ void q4k_half(const int4& h, int hb, u32& sc, u32& mn
         sc = ((u32)h.w & 0x0F0F0F0Fu) | (((u32)h.y >> 2) & 0x30303030u);
         mn = (((u32)h.w >> 4) & 0x0F0F0F0Fu) | (((u32)h.z >> 2) & 0x30303030u);
     }
+    // (Kept whole: folded into its uses, the mask became an AND per byte.)
+    __asm__ volatile("" : "+v"(sc), "+v"(mn));
 }
 
 // Q6_K's fourth window from the dwords of the first three (2-bit pieces into
@@ -242,46 +245,40 @@ struct Dot4Source {
     static __device__ __forceinline__ const char* at(int c, int r, int s) {
         return cols_lds + ((c * ROWS + r) * 8 + ((s & 7) ^ swz(r))) * 16;
     }
+    // Block b's two dwords of half hb. NIB: the low nibbles of a chunk's bytes
+    // are elements 0-15, the high ones 16-31, so k-groups 0 and 2 take the low,
+    // 1 and 3 the high nibbles of its first and second eight bytes. Q8_0: a
+    // chunk per 16 elements. Q6_K: block b of window 2 hb (b < 2) or 2 hb + 1,
+    // window w's blocks in chunks 1 + 4 w .. 4 + 4 w, window 3 gathered from
+    // the three others'.
+    __device__ __forceinline__ void codes(int t, int s, int hb, int b, u32 (&u)[2]) const {
+        const int lane = threadIdx.x & 63, g = lane >> 4, r = 16 * t + (lane & 15);
+        auto get = [&](int c) { return *(const uint2*)(at(c, r, s) + 8 * (g >> 1)); };
+        uint2 v;
+        if constexpr (ColsFmt<FMT>::NIB) {
+            v = get(1 + 4 * hb + b);
+        } else if constexpr (FMT == RQ_FMT_Q8_0) {
+            v = get(1 + 2 * (4 * hb + b) + (g & 1));
+        } else {
+            const int c = 1 + 2 * (b & 1) + (g & 1);
+            if (hb == 0 || b < 2) {
+                v = get(c + 4 * (2 * hb + (b >> 1)));
+            } else {
+                const uint2 x = get(c), y = get(c + 4), z = get(c + 8);
+                v = make_uint2(q6_fourth(x.x, y.x, z.x), q6_fourth(x.y, y.y, z.y));
+            }
+        }
+        u[0] = v.x;
+        u[1] = v.y;
+    }
+    // The half's scales, and (CODES) its blocks' codes; OWN: d of row n alone.
+    template <bool OWN = false, bool CODES = true>
     __device__ __forceinline__ HalfW<FMT> half(int t, int s, int hb) const {
         const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, r = 16 * t + n;
         HalfW<FMT> h;
-        if constexpr (ColsFmt<FMT>::NIB) {
-            // Low nibbles of a chunk's bytes are elements 0-15, high ones
-            // 16-31: k-groups 0 and 2 take the low, 1 and 3 the high nibbles
-            // of its first and second eight bytes.
+        if constexpr (CODES)
 #pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const uint2 v = *(const uint2*)(at(1 + 4 * hb + b, r, s) + 8 * (g >> 1));
-                h.u[b][0] = v.x;
-                h.u[b][1] = v.y;
-            }
-        } else if constexpr (FMT == RQ_FMT_Q8_0) {
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const uint2 v = *(const uint2*)(at(1 + 2 * (4 * hb + b) + (g & 1), r, s) + 8 * (g >> 1));
-                h.u[b][0] = v.x;
-                h.u[b][1] = v.y;
-            }
-        } else {
-            // Window w, block b of it: chunks 1 + 4w + 2b (elements 0-15) and
-            // the next; window 3 gathers from the three windows' chunks.
-#pragma unroll
-            for (int b = 0; b < 2; b++) {
-                u32 w[3][2];
-#pragma unroll
-                for (int i = 0; i < 3; i++) {
-                    if (hb == 0 && i == 2) continue;
-                    const uint2 v = *(const uint2*)(at(1 + 4 * i + 2 * b + (g & 1), r, s) + 8 * (g >> 1));
-                    w[i][0] = v.x;
-                    w[i][1] = v.y;
-                }
-#pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    h.u[b][j] = hb == 0 ? w[0][j] : w[2][j];
-                    h.u[2 + b][j] = hb == 0 ? w[1][j] : q6_fourth(w[0][j], w[1][j], w[2][j]);
-                }
-            }
-        }
+            for (int b = 0; b < 4; b++) codes(t, s, hb, b, h.u[b]);
         if constexpr (FMT == RQ_FMT_Q4_K) {
             const int4 hd = *(const int4*)at(0, r, s);
             q4k_half(hd, hb, h.sc, h.mn);
@@ -293,8 +290,8 @@ struct Dot4Source {
             h.sc6[1] = v.y;
         }
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int re = 16 * t + 4 * g + e;
+        for (int e = 0; e < (OWN ? 1 : 4); e++) {
+            const int re = OWN ? r : 16 * t + 4 * g + e;
             if constexpr (ColsFmt<FMT>::BLOCK_D) {
                 const uint2 v = *(const uint2*)(at(0, re, s) + 8 * hb);
                 h.d[e][0] = v.x;
@@ -346,6 +343,7 @@ struct MfmaSource {
         __asm__ volatile("" : "=v"(hv[t].x), "=v"(hv[t].y), "=v"(hv[t].z), "=v"(hv[t].w));
         if constexpr (FMT == RQ_FMT_Q6_K) __asm__ volatile("" : "=v"(dv[t]));
     }
+    template <bool OWN = false, bool CODES = true>
     __device__ __forceinline__ HalfW<FMT> half(int t, int s, int hb) const {
         (void)s;
         const int lane = threadIdx.x & 63, g = lane >> 4;
@@ -385,6 +383,11 @@ struct MfmaSource {
         if constexpr (FMT == RQ_FMT_Q6_K) {
             h.sc6[0] = dw(hv[t], 2 * hb);
             h.sc6[1] = dw(hv[t], 2 * hb + 1);
+        }
+        if constexpr (OWN) {
+            h.d[0][0] = ColsFmt<FMT>::BLOCK_D ? dw(hv[t], 2 * hb) : FMT == RQ_FMT_Q4_K ? (u32)hv[t].x : dv[t];
+            h.d[0][1] = ColsFmt<FMT>::BLOCK_D ? dw(hv[t], 2 * hb + 1) : 0u;
+            return h;
         }
         // Rows 4 g + e of the tile sit in lanes 4 g + e.
 #pragma unroll
@@ -755,3 +758,272 @@ RQ_COLS_FMT(q8_0, RQ_FMT_Q8_0)
 RQ_COLS_FMT(q4_k, RQ_FMT_Q4_K)
 RQ_COLS_FMT(q6_k, RQ_FMT_Q6_K)
 RQ_COLS_ALL(q4_k_q6_k, RQ_FMT_MIX_K)
+
+// ---------------------------------------------------------------------------
+// The f16 GEMM route for short prompts (rq_gemm_<fmt>_<layout>): out[a][r] =
+// sum over k of f16(x) f16(w), accumulated in f32, with the weights
+// dequantized in registers: no f16 copy of the weight is written and read
+// back (3.6 times a weight's Q4_K bytes, whose 27 us for 14336 x 4096 were
+// half of the call up to a few hundred columns).
+//
+// Same split as the matvecs above: 32 rows and 96 or 128 columns per
+// workgroup, its eight waves on the row's super-blocks in turn, their sums
+// added pairwise. Bound by VALU: a weight operand (32 elements of 16 rows)
+// takes about 38 and is used by six or eight v_mfma_f32_16x16x32_f16 of 16
+// cycles, so fewer columns per workgroup would dequantize more than they
+// multiply, and more rows would leave the chip short of workgroups (64 rows
+// by 64 columns: 14336 x 4096 at 128 columns 45 us against 38). A value is
+// evaluated in f32 and rounded to f16 once, as the dequantization to a copy
+// does. x comes from rq_x16_tiles in the operands' own order: one load per
+// wave, 1 KB contiguous, per block and column group.
+//
+// Us per call of the route, copy + rocBLAS -> these, dot4 / MFMA layout: Q4_K
+// 14336 x 4096 at 96 columns 55.8 -> 34.4 / 62.5 -> 30.5, at 128 59.9 -> 38.0
+// / 64 -> 35.7, at 256 75.5 -> 65.1 / 77 -> 62.1; Q6_K 4096 x 14336 at 128
+// 69 -> 57 / 57; Q4_K 4096 x 4096 at 128 38.8 -> 20.0 / 19.4.
+
+// Block b's weight operand: f16 of the dequantized values.
+template <int FMT, int LAY>
+__device__ __forceinline__ Op value_op(const HalfW<FMT>& h, const u32 (&u)[2], int b, const Masks& mk) {
+    const int g = (threadIdx.x & 63) >> 4;
+    const u32 u0 = u[0], u1 = u[1];
+    // The codes q, exact in f16: as q (Q8_0, Q4_K), q - 8 (Q4_0) or 4 (q - 32)
+    // (Q6_K).
+    Op q;
+    if constexpr (ColsFmt<FMT>::NIB) {
+        // The nibble to bits 7..4 of its byte: 1024 + 16 q.
+        u32 v[2][2];
+        u32 key = 0x64006400u;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            if constexpr (LAY == RQ_LAY_DOT4) {
+                const int sh = 4 * (~g & 1);
+                v[i][0] = u[i] << sh;
+                v[i][1] = u[i] >> (8 - sh);
+                key = 0x64006400u | ((g & 1) ? 0x00800080u : 0u);  // high nibbles are stored XOR 8
+            } else if (b < 2) {
+                v[i][0] = u[i] << 4;
+                v[i][1] = u[i] >> 4;
+            } else {
+                v[i][0] = u[i];
+                v[i][1] = u[i] >> 8;
+                key = 0x64806480u;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            q.r[i] = as_h2((v[i >> 1][i & 1] & mk.high) ^ key);
+            q.r[i] = __builtin_elementwise_fma(q.r[i], splat((_Float16)0.0625f),
+                                               splat((_Float16)(FMT == RQ_FMT_Q4_0 ? -72.f : -64.f)));
+        }
+    } else {
+        q = bytes_op(FMT == RQ_FMT_Q6_K ? u0 & 0xFCFCFCFCu : u0, FMT == RQ_FMT_Q6_K ? u1 & 0xFCFCFCFCu : u1, mk.byte);
+    }
+    if constexpr (ColsFmt<FMT>::BLOCK_D) {
+        // One rounding of the exact product of two f16 values.
+        const float d = half_at(h.d[0][b >> 1], b & 1);
+        Op o;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) o.r[i][j] = (_Float16)((float)q.r[i][j] * d);
+        return o;
+    } else {
+        float s, m = 0.f;
+        if constexpr (FMT == RQ_FMT_Q4_K) {
+            s = half_at(h.d[0][0], 0) * (float)((h.sc >> (8 * b)) & 0xFFu);
+            m = -half_at(h.d[0][0], 1) * (float)((h.mn >> (8 * b)) & 0xFFu);
+        } else {
+            const u32 w = b < 2 ? h.sc6[0] : h.sc6[1];
+            s = half_at(h.d[0][0], 0) * (float)(int8_t)(w >> (8 * (2 * (b & 1) + (g & 1)))) * 0.25f;
+        }
+        Op o;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) o.r[i][j] = (_Float16)fmaf((float)q.r[i][j], s, m);
+        return o;
+    }
+}
+
+template <int FMT, int LAY, int RT, int CG>
+__device__ __forceinline__ void gemm_body(const RqGemmParams& P) {
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, n = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // The column chunks of one row block run on one XCD (workgroups go to the
+    // XCDs in turn), so that its L2 serves all but the first read of the
+    // weights.
+    const int blk = blockIdx.x, per = 8 * P.chunks;
+    const int rb = (blk / per) * 8 + (blk & 7), chunk = (blk % per) >> 3;
+    if (rb >= P.row_blocks) return;
+    ColsRows<RT, false> W;
+    W.t0 = P.t;
+    W.row0 = rb * 16 * RT;
+    RqColsParams C;  // what the weight sources read
+    C.lr = P.lr;
+    C.S = P.S;
+    C.S2 = P.S2;
+    using Source =
+        typename std::conditional<LAY == RQ_LAY_DOT4, Dot4Source<FMT, RT, false>, MfmaSource<FMT, RT, false>>::type;
+    const int S = P.S, nb = P.k >> 5, groups = P.groups;
+    const int g0 = chunk * CG;
+    // Column group g0 + c (past the last: the last again, unused).
+    u32 goff[CG];
+#pragma unroll
+    for (int c = 0; c < CG; c++) goff[c] = (u32)min(g0 + c, groups - 1) * 1024u + lane * 16u;
+    auto xload = [&](int kb, Op (&x)[CG]) {
+        const u8* p = (const u8*)P.x + (int64_t)min(kb, nb - 1) * groups * 1024;
+#pragma unroll
+        for (int c = 0; c < CG; c++) x[c] = __builtin_bit_cast(Op, ld16(p + goff[c]));
+    };
+
+    v4f acc[RT][CG];
+#pragma unroll
+    for (int t = 0; t < RT; t++)
+#pragma unroll
+        for (int c = 0; c < CG; c++) acc[t][c] = v4f{0.f, 0.f, 0.f, 0.f};
+    const Masks mk = masks<FMT>();
+    const int nit = (S + 7) >> 3;
+    const int s0 = min(wave, S - 1);
+    // A block's activations are loaded XN - 1 blocks ahead: one block ahead
+    // left each block waiting on an L2 round trip. (Q6_K and Q8_0 in the dot4
+    // layout hold 13 and 17 chunks of the next weights in registers.)
+    constexpr int XN = (LAY == RQ_LAY_DOT4 && ColsFmt<FMT>::C > 9) || CG > 4 ? 2 : 4;
+    Op x[XN][CG];
+    Source src;
+#pragma unroll
+    for (int i = 0; i < XN - 1; i++) xload(8 * s0 + i, x[i]);
+    src.load(C, W, LAY == RQ_LAY_DOT4 ? 0 : s0);
+
+    for (int it = 0; it < nit; it++) {
+        const int s = 8 * it + wave;
+        if constexpr (LAY == RQ_LAY_DOT4) {
+            if (it > 0) __syncthreads();  // the last super-blocks' reads are done
+            src.store();
+            __syncthreads();
+        }
+        if (s >= S) {  // the wave has no super-block in this step, the last
+            if constexpr (LAY == RQ_LAY_DOT4) continue;  // (to the barriers)
+            break;
+        }
+#pragma unroll
+        for (int hb = 0; hb < 2; hb++) {
+            if (!sgpr_value(1)) continue;
+            // (Dot4 layout: the codes come from LDS block by block.)
+            constexpr bool LATE = LAY == RQ_LAY_DOT4;
+            HalfW<FMT> h[RT];
+            u32 u[2][RT][2];
+#pragma unroll
+            for (int t = 0; t < RT; t++) {
+                h[t] = src.template half<true, !LATE>(t, s, hb);
+                if constexpr (LATE) src.codes(t, s, hb, 0, u[0][t]);
+            }
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                const int kb = 8 * s + 4 * hb + b, ahead = 4 * hb + b + XN - 1;
+                // Past the super-block's end: the wave's next one's blocks.
+                xload(ahead < 8 ? 8 * s + ahead : 8 * min(s + 8, S - 1) + ahead - 8, x[ahead % XN]);
+                if constexpr (LATE) {
+                    if (hb == 0 && b == 0 && it + 1 < nit) src.load(C, W, it + 1);
+                    if (b < 3)
+#pragma unroll
+                        for (int t = 0; t < RT; t++) src.codes(t, s, hb, b + 1, u[(b + 1) & 1][t]);
+                }
+                if (!sgpr_value(1) || kb >= nb) continue;  // (past a partial super-block's end)
+#pragma unroll
+                for (int t = 0; t < RT; t++) {
+                    const Op o = value_op<FMT, LAY>(h[t], LATE ? u[b & 1][t] : h[t].u[b], b, mk);
+#pragma unroll
+                    for (int c = 0; c < CG; c++) acc[t][c] = mfma(o, x[(4 * hb + b) % XN][c], acc[t][c]);
+                }
+            }
+            if constexpr (LAY == RQ_LAY_MFMA)
+                if (hb == 1) {
+#pragma unroll
+                    for (int t = 0; t < RT; t++) {
+                        if (s + 8 < S)
+                            src.load_tile(C, W, t, s + 8);
+                        else
+                            src.drop_tile(t);
+                    }
+                }
+        }
+    }
+
+    // The eight waves' sums, as in cols_body.
+    __syncthreads();
+    v4f* part = (v4f*)cols_lds;
+#pragma unroll
+    for (int t = 0; t < RT; t++)
+#pragma unroll
+        for (int c = 0; c < CG; c++)
+            part[((wave * RT + t) * CG + c) * 64 + 16 * g + (n ^ ((4 * t + g) & 15))] = acc[t][c];
+    __syncthreads();
+    for (int it = tid; it < CG * 16 * 4 * RT; it += RQ_COLS_THREADS) {
+        const int c = it / (4 * RT), q = it % (4 * RT), t = q >> 2, gg = q & 3;
+        const int row = W.row0 + 4 * q, col = 16 * g0 + c;
+        if (col >= P.m || row >= W.t0.n) continue;
+        v4f v[RQ_COLS_PARTS];
+#pragma unroll
+        for (int w = 0; w < RQ_COLS_PARTS; w++)
+            v[w] = part[((w * RT + t) * CG + (c >> 4)) * 64 + 16 * gg + ((c & 15) ^ ((4 * t + gg) & 15))];
+#pragma unroll
+        for (int d = 1; d < RQ_COLS_PARTS; d *= 2)
+#pragma unroll
+            for (int w = 0; w < RQ_COLS_PARTS; w += 2 * d) v[w] += v[w + d];
+        float* o = W.t0.out + (int64_t)col * W.t0.n + row;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (row + e < W.t0.n) gmem(o)[e] = v[0][e];
+    }
+}
+
+#define RQ_GEMM(NAME, FMT, LN, LAY, RT, CG)                                                                        \
+    extern "C" __global__ __launch_bounds__(RQ_COLS_THREADS) void rq_gemm_##NAME##_##LN##_##RT##x##CG(RqGemmParams p) { \
+        gemm_body<FMT, LAY, RT, CG>(p);                                                                            \
+    }
+#define RQ_GEMM_FMT(NAME, FMT)                 \
+    RQ_GEMM(NAME, FMT, d, RQ_LAY_DOT4, 2, 6)   \
+    RQ_GEMM(NAME, FMT, d, RQ_LAY_DOT4, 2, 8)   \
+    RQ_GEMM(NAME, FMT, m, RQ_LAY_MFMA, 2, 6)   \
+    RQ_GEMM(NAME, FMT, m, RQ_LAY_MFMA, 2, 8)
+RQ_GEMM_FMT(q4_0, RQ_FMT_Q4_0)
+RQ_GEMM_FMT(q8_0, RQ_FMT_Q8_0)
+RQ_GEMM_FMT(q4_k, RQ_FMT_Q4_K)
+RQ_GEMM_FMT(q6_k, RQ_FMT_Q6_K)
+
+// x f32 [m][k] -> f16 (round to nearest even) in the operand order of
+// rq_gemm_*: per 32-element block and group of 16 columns (zeros past m) 1 KB,
+// lane 16 g + c holding column c's elements of k-group g (win_of's order, each
+// dword's bytes 0, 2, 1, 3). A workgroup takes 8 blocks of a group: a thread
+// converts 16 consecutive elements, 16 threads a column's 1 KB, and the
+// operands leave through LDS as whole kilobytes. (A thread per lane of the
+// result, reading 32 bytes of each of 16 columns, took 5.1 us for 128 columns
+// of 4096.)
+extern "C" __global__ __launch_bounds__(RQ_THREADS) void rq_x16_tiles(RqX16Params p) {
+    __shared__ int4 lds[8 * 65];  // (a block's 64 pieces and one of skew)
+    const int tid = threadIdx.x, c = tid >> 4, e = tid & 15, kb0 = blockIdx.x / p.groups * 8;
+    const int grp = blockIdx.x - blockIdx.x / p.groups * p.groups;
+    const int kb = kb0 + (e >> 1), col = grp * 16 + c;
+    int4 v[2] = {make_int4(0, 0, 0, 0), make_int4(0, 0, 0, 0)};
+    if (col < p.m && kb < p.nb) {
+        const float* src = p.x + (int64_t)col * 32 * p.nb + 32 * kb + 16 * (e & 1);
+        const auto pair = [](int a, int b) {
+            return (int)((u32)f2h(__int_as_float(a)) | ((u32)f2h(__int_as_float(b)) << 16));
+        };
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int4 a = ld16(src + 8 * i), b = ld16(src + 8 * i + 4);
+            v[i] = make_int4(pair(a.x, a.z), pair(a.y, a.w), pair(b.x, b.z), pair(b.y, b.w));
+        }
+    }
+    // Elements 0-7 and 8-15 of a half block: k-groups e % 2 and 2 + e % 2.
+#pragma unroll
+    for (int i = 0; i < 2; i++) lds[(e >> 1) * 65 + 16 * ((e & 1) + 2 * i) + c] = v[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int b = (tid >> 6) + 4 * i;
+        if (kb0 + b < p.nb) st16(p.y + (((int64_t)(kb0 + b) * p.groups + grp) * 64 + (tid & 63)) * 8, lds[b * 65 + (tid & 63)]);
+    }
+}

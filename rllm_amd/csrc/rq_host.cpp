@@ -270,6 +270,11 @@ struct rq_ctx {
     hipModule_t cols_mod = nullptr;
     hipFunction_t cols[RQ_NUM_FMTS + 1][2][3][RQ_COLS_MAX_GROUPS] = {};
     hipFunction_t colsglu[RQ_NUM_FMTS][2] = {};
+    // The f16 GEMM route's kernels that dequantize in registers, by format,
+    // layout and column groups per workgroup (6, 8), and the kernel that puts x
+    // in their operands' order.
+    hipFunction_t gemm[RQ_NUM_FMTS][2][2] = {};
+    hipFunction_t x16_tiles = nullptr;
     // The f16 GEMM route of batched rq_matmul* (rq_set_gemm_min_m): f16
     // dequantization from either layout, f32 -> f16, rocBLAS (created by the
     // first such call or rq_reserve_f16, with a fixed workspace), and the
@@ -1578,11 +1583,18 @@ extern "C" rq_status rq_open(int device, rq_ctx** out) {
                     snprintf(name, sizeof name, "rq_cols_%s_%c_%dx%d", fs, "dm"[l], rt, cg);
                     st = getm(ctx->cols_mod, &ctx->cols[f][l][rt >> 1][cg - 1], name);
                 }
+        for (int l = 0; l < 2 && f < RQ_NUM_FMTS && st == RQ_OK; l++) {
+            snprintf(name, sizeof name, "rq_gemm_%s_%c_2x6", fs, "dm"[l]);
+            st = getm(ctx->cols_mod, &ctx->gemm[f][l][0], name);
+            snprintf(name, sizeof name, "rq_gemm_%s_%c_2x8", fs, "dm"[l]);
+            if (st == RQ_OK) st = getm(ctx->cols_mod, &ctx->gemm[f][l][1], name);
+        }
         for (int cg = 1; cg <= 2 && f < RQ_NUM_FMTS && st == RQ_OK; cg++) {
             snprintf(name, sizeof name, "rq_colsglu_%s_%d", fs, cg);
             st = getm(ctx->cols_mod, &ctx->colsglu[f][cg - 1], name);
         }
     }
+    if (st == RQ_OK) st = getm(ctx->cols_mod, &ctx->x16_tiles, "rq_x16_tiles");
     if (st != RQ_OK) return bail(st);
     // Defaults and tuning overrides from the environment.
     if (const char* v = getenv("RQ_KERNELS")) {
@@ -2051,6 +2063,7 @@ extern "C" rq_status rq_matvec(rq_ctx* ctx, const rq_q8_1* xq, int64_t m, const 
 namespace {
 rq_status ensure_blas(rq_ctx* ctx);
 rq_status grow_f16(rq_ctx* ctx, uint16_t** p, int64_t* cap, int64_t values);
+int64_t x16_values(int64_t v);
 rq_status dequant16_launch(rq_ctx* ctx, const rq_weight* w, uint16_t* out);
 rq_status refuse_capture(rq_ctx* ctx, const char* what);
 rq_status grow_parts(rq_ctx* ctx, int64_t values);
@@ -2073,7 +2086,7 @@ extern "C" rq_status rq_reserve_f16(rq_ctx* ctx, int64_t weight_values, int64_t 
     if (st != RQ_OK) return st;
     if ((st = ensure_blas(ctx)) != RQ_OK) return st;
     if ((st = grow_f16(ctx, &ctx->w16, &ctx->w16_cap, weight_values)) != RQ_OK) return st;
-    if ((st = grow_f16(ctx, &ctx->x16, &ctx->x16_cap, x_values)) != RQ_OK) return st;
+    if ((st = grow_f16(ctx, &ctx->x16, &ctx->x16_cap, x16_values(x_values))) != RQ_OK) return st;
     if ((st = grow_parts(ctx, kMaxGemmSplits * ((out_values + 3) & ~int64_t(3)))) != RQ_OK) return st;
     return grow_uroute(ctx, out_values);
 }
@@ -2254,16 +2267,90 @@ rq_status dequant16_launch(rq_ctx* ctx, const rq_weight* w, uint16_t* out) {
 // Whether batched matmuls of m columns take the f16 GEMM route.
 bool gemm_route_takes(const rq_ctx* ctx, int64_t m) { return ctx->gemm_min_m > 0 && m >= ctx->gemm_min_m; }
 
+// Rows and columns of an rq_gemm_* workgroup: 32 rows, 6 or 8 groups of 16
+// columns (two launch shapes, so that 96 and 192 columns do not pay for 128
+// and 256).
+constexpr int kGemmTiles = 2;
+int gemm_groups(int64_t m) {
+    const int64_t groups = (m + 15) / 16, chunks = (groups + 7) / 8;
+    return (groups + chunks - 1) / chunks > 6 ? 8 : 6;
+}
+
+// Whether the route's product of w with m columns dequantizes in registers
+// (rq_gemm_*) instead of writing an f16 copy for rocBLAS. The copy costs 27 us
+// for 14336 x 4096, once per call; rocBLAS then takes half as long per column.
+// Up to 256 columns the kernels win (us, copy + rocBLAS -> here, dot4 layout,
+// at 96 / 128 / 256 columns: Q4_K 14336 x 4096 55.8 / 59.9 / 75.5 -> 34.4 /
+// 38.0 / 65.1, 13824 x 5120 64.6 / 68.3 / 90.1 -> 42.7 / 48.8 / 85.2, Q6_K
+// 4096 x 14336 59 / 69 / 78 -> 51 / 57 / 59; at 384 14336 x 4096 80 -> 103),
+// beyond where the chip holds the product in two rounds of workgroups (Q4_K
+// 4096 x 4096 at 512: 44.2 -> 38.6, Q6_K 1024 x 4096 at 1024: 33.5 -> 26.6;
+// four: 4096 x 4096 at 1024 57 -> 79), but from k = 8192 rocBLAS splits k
+// there. A weight with a kept copy has paid for it: rocBLAS is then as fast or
+// faster on the largest shapes (14336 x 4096 at 256: 56.0). Below 65 columns,
+// where only a lowered threshold leads, x in operand order would be padded
+// past what rq_reserve_f16 sizes.
+constexpr int64_t kGemmFusedMinM = 65, kGemmFusedMaxM = 256, kGemmFusedMaxK = 8192;
+bool gemm_fused(const rq_ctx* ctx, const rq_weight* w, int64_t m) {
+    if (w->f16 || m < kGemmFusedMinM) return false;
+    if (m <= kGemmFusedMaxM) return true;
+    const int64_t blocks = (w->rows + 16 * kGemmTiles - 1) / (16 * kGemmTiles);
+    const int64_t per = 16 * gemm_groups(m);
+    return w->cols < kGemmFusedMaxK && blocks * ((m + per - 1) / per) <= 2 * ctx->cus;
+}
+
+// Values of the x scratch for v values of x: in operand order columns are
+// padded to groups of 16, by at most 80 / 65 from kGemmFusedMinM on. Taken for
+// every call of the route, so that a scratch that served one shape serves any
+// other with no more values.
+int64_t x16_values(int64_t v) { return (v * 80 + 64) / 65; }
+
+rq_status gemm_fused_launch(rq_ctx* ctx, const rq_weight* w, int64_t m, float* out) {
+    const bool mfma = w->mmq;
+    const int cg = gemm_groups(m);
+    RqGemmParams p;
+    memset(&p, 0, sizeof p);
+    p.t = cols_target(w, mfma);
+    p.t.out = out;
+    p.x = ctx->x16;
+    p.m = (int32_t)m;
+    p.k = (int32_t)w->cols;
+    p.S = (int32_t)((w->cols + 255) / 256);
+    p.S2 = w->S2;
+    p.lr = mfma ? 0 : log2_of(w->tiled.R);
+    p.groups = (int32_t)((m + 15) / 16);
+    p.chunks = (p.groups + cg - 1) / cg;
+    p.row_blocks = (p.t.tiles + kGemmTiles - 1) / kGemmTiles;
+    // The dot4 layout's staged chunks of eight super-blocks, at the end the
+    // eight waves' sums.
+    const int stage = mfma ? 0 : 16 * kGemmTiles * 8 * (rq_chunks(w->fmt) * 16 + (w->fmt == RQ_FMT_Q6_K ? 2 : 0));
+    const int lds = std::max(stage, RQ_COLS_PARTS * kGemmTiles * cg * 1024);
+    return launch(ctx, ctx->gemm[w->fmt][mfma ? 1 : 0][cg == 8 ? 1 : 0], "rq_gemm",
+                  (uint64_t)((p.row_blocks + 7) / 8 * 8) * p.chunks, &p, (unsigned)lds, RQ_COLS_THREADS);
+}
+
 rq_status gemm_route(rq_ctx* ctx, const float* x, int64_t m, const rq_weight* const* ws, float* const* outs,
                      int count) {
     const int64_t k = ws[0]->cols;
     int64_t wmax = 0;  // the largest weight without a persistent f16 copy
-    for (int i = 0; i < count; i++)
+    int fused = 0;
+    for (int i = 0; i < count; i++) {
         if (!ws[i]->f16) wmax = std::max(wmax, ws[i]->rows * k);
+        fused += gemm_fused(ctx, ws[i], m);
+    }
     rq_status st;
     if ((st = ensure_blas(ctx)) != RQ_OK) return st;
-    if ((st = grow_f16(ctx, &ctx->x16, &ctx->x16_cap, m * k)) != RQ_OK) return st;
+    if ((st = grow_f16(ctx, &ctx->x16, &ctx->x16_cap, x16_values(m * k))) != RQ_OK) return st;
     if ((st = grow_f16(ctx, &ctx->w16, &ctx->w16_cap, wmax)) != RQ_OK) return st;
+    if (fused) {
+        // These first: x in operand order then makes way for row-major x.
+        RqX16Params xp{x, ctx->x16, (int32_t)m, (int32_t)(k / 32), (int32_t)((m + 15) / 16), 0};
+        if ((st = launch(ctx, ctx->x16_tiles, "rq_x16_tiles", (uint64_t)xp.groups * ((xp.nb + 7) / 8), &xp)) != RQ_OK)
+            return st;
+        for (int i = 0; i < count; i++)
+            if (gemm_fused(ctx, ws[i], m) && (st = gemm_fused_launch(ctx, ws[i], m, outs[i])) != RQ_OK) return st;
+        if (fused == count) return RQ_OK;
+    }
     RqConvParams cp{x, ctx->x16, m * k};
     if ((st = launch(ctx, ctx->f2h, "rq_f32_to_f16", (uint64_t)((m * k / 8 + RQ_THREADS - 1) / RQ_THREADS), &cp)) !=
         RQ_OK)
@@ -2273,6 +2360,7 @@ rq_status gemm_route(rq_ctx* ctx, const float* x, int64_t m, const rq_weight* co
     const float alpha = 1.f, beta = 0.f;
     for (int i = 0; i < count; i++) {
         const rq_weight* w = ws[i];
+        if (gemm_fused(ctx, w, m)) continue;
         const uint16_t* a = w->f16;
         if (!a) {
             if ((st = dequant16_launch(ctx, w, ctx->w16)) != RQ_OK) return st;

@@ -256,6 +256,25 @@ struct RqColsParams {
     uint16_t* hs;
 };
 
+// The f16 GEMM route's kernels that dequantize in registers (rq_gemm_* in
+// rq_cols.hip), rt tiles of 16 rows and cg groups of 16 columns per workgroup.
+struct RqGemmParams {
+    RqColsTarget t;      // out[a * n + r]
+    const uint16_t* x;   // f16 columns in operand order (rq_x16_tiles)
+    int32_t m, k, S, S2, lr;
+    int32_t groups;      // 16-column groups of x, ceil(m / 16)
+    int32_t chunks;      // column chunks of cg groups
+    int32_t row_blocks;  // row blocks of rt tiles
+};
+
+// f32 [m][k] -> f16 operand order (rq_x16_tiles), groups * nb KB.
+struct RqX16Params {
+    const float* x;
+    uint16_t* y;
+    int32_t m, nb;       // columns, 32-element blocks per column
+    int32_t groups, pad;
+};
+
 struct RqMmqRepackParams {
     const uint8_t* raw;  // GGUF bytes of rows [row0, row0 + rows)
     uint8_t* code;

@@ -1,0 +1,90 @@
+"""The f16 GEMM route's kernels that dequantize in registers (rq_gemm_*), at
+the edges of their row blocks, column groups and super-blocks: against the
+exact product of the f16 values, both layouts bit-identical, and beside
+weights that stay with the vendor GEMM."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import make_weight, upload
+
+pytestmark = pytest.mark.gpu
+
+TYPES = {"Q4_0": 2, "Q8_0": 8, "Q4_K": 12, "Q6_K": 14}
+
+# Against f64 over both operands rounded to f16. f32 sums as in the matvecs:
+# within 1e-5 of the largest output. A K-quant value whose f32 lies within its
+# rounding of an f16 tie (one in 2^11 or fewer) may round the other way, 2^-11
+# of one term: at k >= 256 and outputs of several row norms, 1e-5 each if it
+# hits the largest output's row; four of them aligned.
+TOL = 5e-5
+
+
+def _exact(orc, t, w, n, k, x, m):
+    f16 = lambda v: v.astype(np.float16).astype(np.float64)
+    return (f16(x.reshape(m, k)) @ f16(orc.dequantize(t, w, n, k).reshape(n, k)).T).reshape(-1)
+
+
+@pytest.mark.parametrize("tname", list(TYPES))
+@pytest.mark.parametrize("n,k", [(1, 256), (17, 2048), (32, 2304), (70, 4096), (300, 14336), (33, 32), (50, 2080)])
+@pytest.mark.parametrize("m", [65, 96, 97, 128, 129, 192, 193, 256, 500])
+def test_gemm_fused(gpu, orc, tname, n, k, m):
+    t = TYPES[tname]
+    if t in (12, 14) and k % 256:
+        pytest.skip("K-quants need k % 256 == 0")
+    w = make_weight(orc, t, n, k, 60 + n, "normal")
+    x = orc.normal(61 + k + m, m * k, 0.0, 1.0)
+    xg = gpu.from_host(x)
+    want, got = _exact(orc, t, w, n, k, x, m), {}
+    for fam in ("dot4", "mfma"):
+        gpu.set_kernels(fam)
+        wg = upload(gpu, t, w, n, k)
+        gpu.set_kernels("auto")
+        out = gpu.alloc(m * n + 8)
+        out.fill_(float("nan"))
+        gpu.matmul(xg, wg, out, m)
+        got[fam] = gpu.to_host(out)
+        assert np.isnan(got[fam][m * n:]).all(), "wrote past the output"
+        orc.assert_close(f"{tname} {n}x{k} m={m} {fam}", want, got[fam][:m * n], TOL)
+    if m <= 256 or k < 8192:  # (past them: the vendor GEMM on the copy)
+        assert np.array_equal(got["dot4"][:m * n].view(np.uint32), got["mfma"][:m * n].view(np.uint32))
+
+
+@pytest.mark.parametrize("m", [65, 100])
+@pytest.mark.parametrize("k", [4096, 14336])
+def test_gemm_fused_beside_kept_copies(gpu, orc, k, m):
+    """matmul_many over weights on both sides of the rule (a weight with a kept
+    copy goes to the vendor GEMM, at k = 14336 in slices of k): each as in its
+    own call, and replayed from a graph after reserve_f16."""
+    t, rows = 12, (200, 300, 72)
+    ws = [make_weight(orc, t, n, k, 70 + n, "normal") for n in rows]
+    wgs = [upload(gpu, t, w, n, k) for w, n in zip(ws, rows)]
+    gpu.keep_f16(wgs[1])
+    x = orc.normal(71 + m, m * k, 0.0, 1.0)
+    gpu.reserve_f16(max(rows) * k, m * k, m * max(rows))
+    xg = gpu.from_host(x)
+    own = [gpu.alloc(m * n) for n in rows]
+    for wg, out in zip(wgs, own):
+        gpu.matmul(xg, wg, out, m)
+    for w, n, out in zip(ws, rows, own):
+        orc.assert_close(f"{n}x{k} m={m}", _exact(orc, t, w, n, k, x, m), gpu.to_host(out), TOL)
+    outs = [gpu.alloc(m * n) for n in rows]
+    gpu.matmul_many(xg, wgs, outs, m)
+    gpu.synchronize()
+    for a, b in zip(own, outs):
+        assert torch.equal(a, b)
+    graph, stream, main = torch.cuda.CUDAGraph(), torch.cuda.Stream(gpu.device), gpu.stream
+    torch.cuda.synchronize()
+    gpu.set_stream(stream)
+    try:
+        with torch.cuda.graph(graph, stream=stream):
+            gpu.matmul_many(xg, wgs, outs, m)
+    finally:
+        gpu.set_stream(main)
+    for _ in range(3):
+        for b in outs:
+            b.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(own, outs):
+            assert torch.equal(a, b)
