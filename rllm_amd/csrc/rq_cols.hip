@@ -1,5 +1,5 @@
 // Matvecs over more than 8 activation columns (rq_cols_*, either weight
-// layout, rq_params.h) and the fused gate/up front half of a gated FFN from 6
+// layout, rq_params.h) and the fused gate/up front half of a gated FFN
 // (rq_colsglu_*, the dot4 layout); on the same weight sources the f16 GEMM
 // route's kernels for short prompts (rq_gemm_*, at the end). Which calls come
 // here, and both sides' times: use_cols and gemm_fused in rq_host.cpp.

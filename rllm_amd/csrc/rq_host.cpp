@@ -1141,10 +1141,11 @@ rq_status cols_launch(rq_ctx* ctx, const int8_t* xq, const uint16_t* xd, int64_t
 }
 
 // Gate and up of one type and shape in the dot4 layout through rq_colsglu_*:
-// from 6 columns (Q4_K 14336 x 4096 at 6: 34.0 us in rq_glu_*, 32.1 here; at
-// 16 two launches there).
+// from 9 columns, where rq_glu_* takes a second launch over the weights. At
+// eight and below its one launch stays: the column kernels gain 6 % at most
+// (Q4_K 14336 x 4096 at 6: 34.0 us there, 32.1 here).
 bool cols_glu_ok(const rq_ctx* ctx, const rq_weight* gate, const rq_weight* up, int64_t m) {
-    return m >= 6 && glu_fusable(gate, up, m) &&
+    return m > 8 && glu_fusable(gate, up, m) &&
            cols_glu_groups(ctx, gate->fmt, (int)((gate->cols + 255) / 256)) > 0;
 }
 

@@ -1,5 +1,5 @@
 """The column kernels (rq_cols_*, rq_colsglu_*): matvecs over more than 8
-Q8_1 columns, and the dot4 layout's fused gate/up from 6, against the integer
+Q8_1 columns, and the dot4 layout's fused gate/up from 9, against the integer
 oracle at the edges of their tiles, column groups and rows."""
 import numpy as np
 import pytest
@@ -99,7 +99,7 @@ def test_cols_mixed_launch(gpu, orc, family, k):
 
 @pytest.mark.parametrize("tname", list(TYPES))
 @pytest.mark.parametrize("f,d", [(32, 512), (96, 4096), (64, 5120)])
-@pytest.mark.parametrize("m", [5, 6, 16, 17, 33, 50])
+@pytest.mark.parametrize("m", [8, 9, 16, 17, 33, 50])
 def test_cols_gated_ffn(gpu, orc, tname, f, d, m):
     """The dot4 layout's fused front half: h within 1e-3 of the integer path
     (the activation's expf), the down projection on exactly h's Q8_1."""
