@@ -169,7 +169,7 @@ rq_status rq_matvec(rq_ctx* ctx, const rq_q8_1* xq, int64_t m, const rq_weight* 
  * mixed (q/k/v of a Q4_K_M file), and run by one kernel family at this m
  * (a dot4 weight with an MFMA one fails with RQ_ERR_SHAPE). Each output is
  * bit-identical to the weight's own rq_matvec, except a Q4_K weight of a
- * Q4_K / Q6_K mix on MFMA weights over more than 8 columns: the mixed launch
+ * Q4_K / Q6_K mix on MFMA weights over 9 to 16 columns: the mixed launch
  * runs the 8-column kernels, the weight's own launch the 16-column ones
  * (another summation order, both within the integer path's bound).
  * out_lens[i] >= m * rows_i. */

@@ -2,7 +2,8 @@
 
 1. hipcc --genco compiles each kernel source (csrc/rq_kernels.hip: the Q8_1
    pass and the dot4 matvecs; csrc/rq_mmq.hip: the int8-MFMA matvecs;
-   csrc/rq_cols.hip: the matvecs over 4 to 64 columns) into one gfx950 code
+   csrc/rq_cols.hip: the matvecs over more columns than the
+   dot4 kernels take and the f16 products of short prompts) into one gfx950 code
    object each.
 2. An assembler stub (.incbin) embeds the code objects in the library.
 3. hipcc compiles csrc/rq_static.hip (the fixed device scratch of

@@ -768,11 +768,17 @@ RQ_COLS_ALL(q4_k_q6_k, RQ_FMT_MIX_K)
 //
 // Same split as the matvecs above: 32 rows and 96 or 128 columns per
 // workgroup, its eight waves on the row's super-blocks in turn, their sums
-// added pairwise. Bound by VALU: a weight operand (32 elements of 16 rows)
-// takes about 38 and is used by six or eight v_mfma_f32_16x16x32_f16 of 16
-// cycles, so fewer columns per workgroup would dequantize more than they
-// multiply, and more rows would leave the chip short of workgroups (64 rows
-// by 64 columns: 14336 x 4096 at 128 columns 45 us against 38). A value is
+// added pairwise. A weight operand (32 elements of 16 rows) takes about 38
+// VALU and is used by six or eight v_mfma_f32_16x16x32_f16 of 16 cycles, so
+// fewer columns per workgroup would dequantize more than they multiply, and
+// more rows would leave the chip short of workgroups (64 rows by 64 columns:
+// 14336 x 4096 at 128 columns 45 us against 38). What is left is bound by the
+// reads of x, 1 KB per wave and two products (448 MB from L2 for 14336 x 4096
+// at 128 columns, 12 TB/s), not by VALU or by the loads in flight: 16 % fewer
+// VALU instructions took 1 to 3 % off some shapes and put as much on others
+// (128 columns 36.5 -> 35.9 us, 96 30.6 -> 31.4), and loads two to four
+// blocks ahead on top gained 5 % at most (Q6_K 4096 x 14336 at 128: 57.4 ->
+// 54.7) and lost up to 10 (Q4_0 11008 x 4096 at 96: 29.3 -> 32.2). A value is
 // evaluated in f32 and rounded to f16 once, as the dequantization to a copy
 // does. x comes from rq_x16_tiles in the operands' own order: one load per
 // wave, 1 KB contiguous, per block and column group.

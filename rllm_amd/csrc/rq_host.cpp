@@ -30,7 +30,7 @@
 
 extern "C" const unsigned char rq_kernels_blob[];  // rq_kernels.hip: Q8_1 pass, dot4 matvecs
 extern "C" const unsigned char rq_mmq_blob[];      // rq_mmq.hip: int8-MFMA matvecs
-extern "C" const unsigned char rq_cols_blob[];     // rq_cols.hip: matvecs over 4 to 64 columns
+extern "C" const unsigned char rq_cols_blob[];     // rq_cols.hip: matvecs over 7 to 64 columns, f16 products
 // rq_static.hip: the device address of the fixed scratch of
 // rq_matmul_many_noalloc on the current device.
 extern "C" __attribute__((visibility("hidden"))) hipError_t rq_noalloc_scratch(int device, void** ptr, size_t* bytes);
