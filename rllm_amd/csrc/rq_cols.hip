@@ -826,7 +826,7 @@ __device__ __forceinline__ Op value_op(const HalfW<FMT>& h, const u32 (&u)[2], i
         q = bytes_op(FMT == RQ_FMT_Q6_K ? u0 & 0xFCFCFCFCu : u0, FMT == RQ_FMT_Q6_K ? u1 & 0xFCFCFCFCu : u1, mk.byte);
     }
     if constexpr (ColsFmt<FMT>::BLOCK_D) {
-        // One rounding of the exact product of two f16 values.
+        // One rounding of the exact product of a code and an f16 scale.
         const float d = half_at(h.d[0][b >> 1], b & 1);
         Op o;
 #pragma unroll
@@ -847,7 +847,21 @@ __device__ __forceinline__ Op value_op(const HalfW<FMT>& h, const u32 (&u)[2], i
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
-            for (int j = 0; j < 2; j++) o.r[i][j] = (_Float16)fmaf((float)q.r[i][j], s, m);
+            for (int j = 0; j < 2; j++) {
+                // Q6_K: an exact product. Q4_K: d sc q and dmin m are exact,
+                // their difference need not be, and the copy rounds it to f32
+                // and then to f16: the f32 value passes the empty asm, as in
+                // pack32_f16, or part of the values become v_fma_mix to f16,
+                // one rounding (another value where the f32 is an f16 tie).
+                float v;
+                if constexpr (FMT == RQ_FMT_Q4_K) {
+                    v = fmaf((float)q.r[i][j], s, m);
+                    __asm__ volatile("" : "+v"(v));
+                } else {
+                    v = (float)q.r[i][j] * s;
+                }
+                o.r[i][j] = (_Float16)v;
+            }
         return o;
     }
 }

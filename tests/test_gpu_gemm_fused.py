@@ -12,11 +12,9 @@ pytestmark = pytest.mark.gpu
 
 TYPES = {"Q4_0": 2, "Q8_0": 8, "Q4_K": 12, "Q6_K": 14}
 
-# Against f64 over both operands rounded to f16. f32 sums as in the matvecs:
-# within 1e-5 of the largest output. A K-quant value whose f32 lies within its
-# rounding of an f16 tie (one in 2^11 or fewer) may round the other way, 2^-11
-# of one term: at k >= 256 and outputs of several row norms, 1e-5 each if it
-# hits the largest output's row; four of them aligned.
+# Against f64 over both operands rounded to f16, the very values the kernels
+# multiply (test_gemm_fused_weights_are_the_copys): what is left are the f32
+# sums, within 1e-5 of the largest output as in the matvecs; five times that.
 TOL = 5e-5
 
 
@@ -88,3 +86,43 @@ def test_gemm_fused_beside_kept_copies(gpu, orc, k, m):
         torch.cuda.synchronize()
         for a, b in zip(own, outs):
             assert torch.equal(a, b)
+
+
+def _one_hot(gpu, k, m, first):
+    """m columns, column j one-hot at element first + j (zeros past k)."""
+    x = torch.zeros((m, k), dtype=torch.float32, device=gpu.device)
+    for j in range(min(m, k - first)):
+        x[j, first + j] = 1.0
+    return x
+
+
+@pytest.mark.parametrize("family", ["dot4", "mfma"])
+@pytest.mark.parametrize("m", [96, 128])
+@pytest.mark.parametrize("tname", list(TYPES))
+def test_gemm_fused_weights_are_the_copys(gpu, orc, tname, family, m):
+    """The f16 weights made in registers are those of the dequantized copy
+    (rq_dequant_f16), bit for bit: a one-hot column's product is one weight.
+    Q4_K's super-blocks hold f16 ties: d sc q has 12 significant bits, the last
+    one set, and dmin m is less than half a unit of it in f32, so that the f32
+    difference is the tie and rounds to even, where rounded once from the exact
+    difference it would go down."""
+    t, n, k = TYPES[tname], 64, 256
+    w = make_weight(orc, t, n, k, 80, "random")
+    if t == 12:
+        b = w.reshape(n, 144)
+        odd = np.random.default_rng(81).integers(512, 1024, n) * 2 + 1  # 11 bits, odd
+        b[:, 0:2] = (odd.astype(np.float32) * 2.0 ** -9).astype(np.float16).view(np.uint8).reshape(n, 2)  # d in 2..4
+        b[:, 2:4] = np.full((n, 1), 2.0 ** -24, np.float16).view(np.uint8)  # dmin: the least f16
+        b[:, 4:16] = np.array([1] * 8 + [0x11] * 4, np.uint8)  # every scale and min 1
+    gpu.set_kernels(family)
+    wg = upload(gpu, t, w, n, k)
+    gpu.set_kernels("auto")
+    want = gpu.dequant_f16(wg).reshape(n, k).float()
+    got = torch.empty((n, k), device=gpu.device)
+    for first in range(0, k, m):
+        out = gpu.alloc(m * n)
+        gpu.matmul(_one_hot(gpu, k, m, first).reshape(-1), wg, out, m)
+        cols = min(m, k - first)
+        got[:, first:first + cols] = out[:m * n].reshape(m, n)[:cols].t()
+    bad = int((got != want).sum())
+    assert bad == 0, f"{bad} of {n * k} weights differ"
