@@ -2333,14 +2333,16 @@ rq_status gemm_fused_launch(rq_ctx* ctx, const rq_weight* w, int64_t m, float* o
 rq_status gemm_route(rq_ctx* ctx, const float* x, int64_t m, const rq_weight* const* ws, float* const* outs,
                      int count) {
     const int64_t k = ws[0]->cols;
-    int64_t wmax = 0;  // the largest weight without a persistent f16 copy
-    int fused = 0;
+    int64_t wmax = 0;  // the largest weight to copy
+    int fused = 0;     // weights that take neither copy nor rocBLAS
     for (int i = 0; i < count; i++) {
-        if (!ws[i]->f16) wmax = std::max(wmax, ws[i]->rows * k);
-        fused += gemm_fused(ctx, ws[i], m);
+        if (gemm_fused(ctx, ws[i], m))
+            fused++;
+        else if (!ws[i]->f16)
+            wmax = std::max(wmax, ws[i]->rows * k);
     }
     rq_status st;
-    if ((st = ensure_blas(ctx)) != RQ_OK) return st;
+    if (fused < count && (st = ensure_blas(ctx)) != RQ_OK) return st;
     if ((st = grow_f16(ctx, &ctx->x16, &ctx->x16_cap, x16_values(m * k))) != RQ_OK) return st;
     if ((st = grow_f16(ctx, &ctx->w16, &ctx->w16_cap, wmax)) != RQ_OK) return st;
     if (fused) {

@@ -7,6 +7,8 @@ import pytest
 import torch
 
 from gpu_util import make_weight, upload
+from rllm_amd.backend import HipBackend
+from rllm_amd.errors import ShapeError
 
 pytestmark = pytest.mark.gpu
 
@@ -126,3 +128,48 @@ def test_gemm_fused_weights_are_the_copys(gpu, orc, tname, family, m):
         got[:, first:first + cols] = out[:m * n].reshape(m, n)[:cols].t()
     bad = int((got != want).sum())
     assert bad == 0, f"{bad} of {n * k} weights differ"
+
+
+@pytest.mark.filterwarnings("ignore:The CUDA Graph is empty")
+def test_gemm_fused_takes_no_copy_scratch(gpu, orc):
+    """A call whose weights are all dequantized in registers needs x's scratch
+    alone: no f16 copy of a weight (32 MB here) and no vendor workspace (64
+    MB), and it can be captured with nothing reserved for a weight."""
+    t, n, k, m = 12, 4096, 4096, 100
+    w = orc.random_weight(82, t, n, k)
+    fresh = HipBackend(gpu.device.index or 0)
+    try:
+        wg = upload(fresh, t, w, n, k)
+        x = fresh.from_host(orc.normal(83, m * k, 0.0, 1.0))
+        out = fresh.alloc(m * n)
+        graph, stream, main = torch.cuda.CUDAGraph(), torch.cuda.Stream(fresh.device), fresh.stream
+
+        def capture():
+            torch.cuda.synchronize()
+            fresh.set_stream(stream)
+            try:
+                with torch.cuda.graph(graph, stream=stream):
+                    fresh.matmul(x, wg, out, m)
+            finally:
+                fresh.set_stream(main)
+
+        with pytest.raises(ShapeError, match="rq_reserve_f16"):
+            capture()
+        torch.cuda.synchronize()
+        free0, _ = torch.cuda.mem_get_info(fresh.device)
+        fresh.matmul(x, wg, out, m)
+        fresh.synchronize()
+        free1, _ = torch.cuda.mem_get_info(fresh.device)
+        assert free0 - free1 < 16 << 20, f"the call took {free0 - free1} bytes"
+        want = out.clone()
+        graph = torch.cuda.CUDAGraph()
+        capture()
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want)
+        del graph
+    finally:
+        fresh.synchronize()
+        fresh.close()
