@@ -2303,8 +2303,10 @@ bool gemm_fused(const rq_ctx* ctx, const rq_weight* w, int64_t m) {
 // Values of the x scratch for v values of x: in operand order columns are
 // padded to groups of 16, by at most 80 / 65 from kGemmFusedMinM on. Taken for
 // every call of the route, so that a scratch that served one shape serves any
-// other with no more values.
-int64_t x16_values(int64_t v) { return (v * 80 + 64) / 65; }
+// other with no more values. (Sizes past any memory stay as they are: the
+// product would overflow, and they have to reach the allocator that refuses
+// them.)
+int64_t x16_values(int64_t v) { return v > INT64_MAX / 80 - 1 ? v : (v * 80 + 64) / 65; }
 
 rq_status gemm_fused_launch(rq_ctx* ctx, const rq_weight* w, int64_t m, float* out) {
     const bool mfma = w->mmq;

@@ -8,7 +8,7 @@ import torch
 
 from gpu_util import make_weight, upload
 from rllm_amd.backend import HipBackend
-from rllm_amd.errors import ShapeError
+from rllm_amd.errors import BackendError, ShapeError
 
 pytestmark = pytest.mark.gpu
 
@@ -172,4 +172,17 @@ def test_gemm_fused_takes_no_copy_scratch(gpu, orc):
         del graph
     finally:
         fresh.synchronize()
+        fresh.close()
+
+
+def test_reserve_f16_refuses_more_than_there_is(gpu):
+    """Reservations past any memory fail in the allocator, also where the
+    padded size of x's scratch would not fit 64 bits."""
+    fresh = HipBackend(gpu.device.index or 0)
+    try:
+        for values in (1 << 50, (1 << 63) // 80 + 1, 1 << 60):
+            with pytest.raises(BackendError):
+                fresh.reserve_f16(0, values, 0)
+        fresh.reserve_f16(0, 4096, 0)
+    finally:
         fresh.close()
