@@ -183,6 +183,8 @@ def test_reserve_f16_refuses_more_than_there_is(gpu):
         for values in (1 << 50, (1 << 63) // 80 + 1, 1 << 60):
             with pytest.raises(BackendError):
                 fresh.reserve_f16(0, values, 0)
+            torch.zeros(1, device=fresh.device).add_(1)  # the failure is the library's alone
+            torch.cuda.synchronize()
         fresh.reserve_f16(0, 4096, 0)
     finally:
         fresh.close()
