@@ -2225,15 +2225,19 @@ rq_status grow_uroute(rq_ctx* ctx, int64_t values) {
 // 79.5 -> 43.0 us at m = 128, 113 -> 90 us at m = 512). At k = 4096
 // splitting measured slower (14336 x 4096 at m = 64: 30.4 -> 38.6 us with 2
 // slices). Each slice is a multiple of 64 values.
-int gemm_splits(const rq_ctx* ctx, int64_t rows, int64_t m, int64_t k) {
+int gemm_split_count(int64_t rows, int64_t m, int64_t k) {
     int S = 1;
-    if (ctx->gemm_splits > 0) {
-        S = ctx->gemm_splits;
-    } else if (k >= 8192) {
+    if (k >= 8192) {
         const int64_t blocks = ((rows + 255) / 256) * ((m + 127) / 128);
         S = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxGemmSplits, 256 / blocks));
         while (S > 1 && k / S < 1792) S--;
     }
+    while (S > 1 && k % (64 * S) != 0) S--;
+    return S;
+}
+int gemm_splits(const rq_ctx* ctx, int64_t rows, int64_t m, int64_t k) {
+    if (ctx->gemm_splits <= 0) return gemm_split_count(rows, m, k);
+    int S = ctx->gemm_splits;
     while (S > 1 && k % (64 * S) != 0) S--;
     return S;
 }
@@ -2281,26 +2285,44 @@ int gemm_groups(int64_t m) {
 }
 
 // Whether the route's product of w with m columns dequantizes in registers
-// (rq_gemm_*) instead of writing an f16 copy for rocBLAS. The copy costs 27 us
-// for 14336 x 4096, once per call; rocBLAS then takes half as long per column.
-// Up to 256 columns the kernels win (us, copy + rocBLAS -> here, dot4 layout,
-// at 96 / 128 / 256 columns: Q4_K 14336 x 4096 55.8 / 59.9 / 75.5 -> 34.4 /
-// 38.0 / 65.1, 13824 x 5120 64.6 / 68.3 / 90.1 -> 42.7 / 48.8 / 85.2, Q6_K
-// 4096 x 14336 59 / 69 / 78 -> 51 / 57 / 59; at 384 14336 x 4096 80 -> 103),
-// beyond where the chip holds the product in two rounds of workgroups (Q4_K
-// 4096 x 4096 at 512: 44.2 -> 38.6, Q6_K 1024 x 4096 at 1024: 33.5 -> 26.6;
-// four: 4096 x 4096 at 1024 57 -> 79), but from k = 8192 rocBLAS splits k
-// there. A weight with a kept copy has paid for it: rocBLAS is then as fast or
-// faster on the largest shapes (14336 x 4096 at 256: 56.0). Below 65 columns,
-// where only a lowered threshold leads, x in operand order would be padded
-// past what rq_reserve_f16 sizes.
+// (rq_gemm_*) instead of writing an f16 copy for rocBLAS: where its estimated
+// time is the lower one. Neither side leads everywhere (us, copy + rocBLAS /
+// here, Q4_K, dot4 layout: 4096 x 4096 at 128 columns 39.8 / 21.1, 14336 x
+// 4096 at 128 59 / 41, at 400 90 / 131; 96 x 14336 at 65 18.8 / 43.9, 1024 x
+// 14336 at 128 30.8 / 54.0, 28672 x 512 at 256 37 / 54, 28672 x 2304 at 256
+// 73 / 104).
+//   Here: the conversion of x, then rounds of one workgroup per CU, each of
+//   them one step per eight super-blocks of the row (a step costs its latency
+//   however few of the eight waves have a super-block) and the super-blocks'
+//   products; many rounds of short rows cost an eighth to a fifth more.
+//   Copy + rocBLAS: two launches and the GEMM's latency, the copy (per weight
+//   value), x (per value), the products, a k-slice's length and the output;
+//   an eighth more where rows are not whole 128 values.
+// Fits of the relative error over 13756 calls (96 to 28672 rows, 512 to 14336
+// columns, 65 to 1024 tokens, all types and layouts). Of the 9994 that may
+// come here the choice is more than 3 % slower than copy + rocBLAS in 2 % and
+// than these kernels in 6 %. (By the layout it would be closer, the MFMA one's
+// steps take 1.8 and the dot4 one's 2.6 us, but a product's bits are the same
+// in both.) A weight with a kept copy has paid for it and stays
+// with rocBLAS. Below 65 columns, where only a lowered threshold leads, x in
+// operand order would be padded past what rq_reserve_f16 sizes; past 256
+// columns, where rocBLAS' half the time per column outweighs its copy on any
+// larger weight, only up to two rounds and k < 8192 (rocBLAS splits k there).
 constexpr int64_t kGemmFusedMinM = 65, kGemmFusedMaxM = 256, kGemmFusedMaxK = 8192;
 bool gemm_fused(const rq_ctx* ctx, const rq_weight* w, int64_t m) {
     if (w->f16 || m < kGemmFusedMinM) return false;
-    if (m <= kGemmFusedMaxM) return true;
-    const int64_t blocks = (w->rows + 16 * kGemmTiles - 1) / (16 * kGemmTiles);
-    const int64_t per = 16 * gemm_groups(m);
-    return w->cols < kGemmFusedMaxK && blocks * ((m + per - 1) / per) <= 2 * ctx->cus;
+    const int64_t n = w->rows, k = w->cols, cg = gemm_groups(m), chunks = (m + 16 * cg - 1) / (16 * cg);
+    const int64_t blocks = (n + 16 * kGemmTiles - 1) / (16 * kGemmTiles);
+    if (m > kGemmFusedMaxM && (k >= kGemmFusedMaxK || blocks * chunks > 2 * ctx->cus)) return false;
+    const double mk = 1e-6 * m * k, mn = 1e-6 * m * n, nk = 1e-6 * n * k;
+    const int64_t S = (k + 255) / 256, steps = (S + 7) / 8;
+    const int64_t rounds = ((blocks + 7) / 8 * 8 * chunks + ctx->cus - 1) / ctx->cus;
+    const bool dear = w->fmt == RQ_FMT_Q8_0 || w->fmt == RQ_FMT_Q6_K;  // 13, 17 chunks of weights
+    double own = 3.7 + 1.5 * mk + rounds * (3.5 + cg / 8.0 * (2.3 * steps + (dear ? 0.64 : 0.52) * S));
+    if (rounds > 4 && S <= 16) own *= S <= 12 ? 1.2 : 1.12;
+    double copy = 12.6 + 0.73 * nk + 2.1 * mk + 1.19e-3 * m * nk + 0.74e-3 * k / gemm_split_count(n, m, k) + 1.2 * mn;
+    if (k % 128 != 0) copy *= 1.12;
+    return own < copy;
 }
 
 // Values of the x scratch for v values of x: in operand order columns are

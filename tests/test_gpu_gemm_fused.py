@@ -188,3 +188,20 @@ def test_reserve_f16_refuses_more_than_there_is(gpu):
         fresh.reserve_f16(0, 4096, 0)
     finally:
         fresh.close()
+
+
+@pytest.mark.parametrize("tname", ["Q4_K", "Q8_0"])
+@pytest.mark.parametrize("n,k,m", [(96, 14336, 65), (1024, 14336, 128), (2048, 14336, 112), (1024, 8192, 200),
+                                   (28672, 512, 256), (14336, 512, 200), (96, 6144, 400)])
+def test_gemm_fused_leaves_what_the_copy_does_faster(gpu, orc, tname, n, k, m):
+    """Few rows of many super-blocks, and many rows of few: such products stay
+    with the copy and the vendor GEMM, and so have the bits of a kept copy."""
+    t = TYPES[tname]
+    wg = upload(gpu, t, orc.random_weight(84, t, n, k), n, k)
+    x = gpu.from_host(orc.normal(85, m * k, 0.0, 1.0))
+    got, want = gpu.alloc(m * n), gpu.alloc(m * n)
+    gpu.matmul(x, wg, got, m)
+    gpu.keep_f16(wg)
+    gpu.matmul(x, wg, want, m)
+    assert torch.equal(got, want)
+    wg.free()
