@@ -2296,12 +2296,13 @@ int gemm_groups(int64_t m) {
 //   however few of the eight waves have a super-block) and the super-blocks'
 //   products; many rounds of short rows cost an eighth to a fifth more.
 //   Copy + rocBLAS: two launches and the GEMM's latency, the copy (per weight
-//   value), x (per value), the products, a k-slice's length and the output;
-//   an eighth more where rows are not whole 128 values.
-// Fits of the relative error over 13756 calls (96 to 28672 rows, 512 to 14336
-// columns, 65 to 1024 tokens, all types and layouts). Of the 9994 that may
-// come here the choice is more than 3 % slower than copy + rocBLAS in 2 % and
-// than these kernels in 6 %. (By the layout it would be closer, the MFMA one's
+//   value), x (per value), the products, the GEMM's chain over a k-slice
+//   (shorter tiles below 512 rows), the output and the slices' sum; an eighth
+//   more where rows are not whole 128 values.
+// Fits of the relative error over 26760 calls (96 to 28672 rows, 512 to 14336
+// columns, 65 to 1024 tokens, all types and layouts). Where a call may come
+// here the choice is more than 3 % slower than copy + rocBLAS in 2 % and than
+// these kernels in 3 % of them. (By the layout it would be closer, the MFMA one's
 // steps take 1.8 and the dot4 one's 2.6 us, but a product's bits are the same
 // in both.) A weight with a kept copy has paid for it and stays
 // with rocBLAS. Below 65 columns, where only a lowered threshold leads, x in
@@ -2320,7 +2321,9 @@ bool gemm_fused(const rq_ctx* ctx, const rq_weight* w, int64_t m) {
     const bool dear = w->fmt == RQ_FMT_Q8_0 || w->fmt == RQ_FMT_Q6_K;  // 13, 17 chunks of weights
     double own = 3.7 + 1.5 * mk + rounds * (3.5 + cg / 8.0 * (2.3 * steps + (dear ? 0.64 : 0.52) * S));
     if (rounds > 4 && S <= 16) own *= S <= 12 ? 1.2 : 1.12;
-    double copy = 12.6 + 0.73 * nk + 2.1 * mk + 1.19e-3 * m * nk + 0.74e-3 * k / gemm_split_count(n, m, k) + 1.2 * mn;
+    const int splits = gemm_split_count(n, m, k);
+    double copy = 12 + 0.7 * nk + 1.75 * mk + 1.02e-3 * m * nk + (n <= 512 ? 0.9e-3 : 1.55e-3) * k / splits + 1.9 * mn;
+    if (splits > 1) copy += 6.7;
     if (k % 128 != 0) copy *= 1.12;
     return own < copy;
 }
