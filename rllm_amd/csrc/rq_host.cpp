@@ -249,7 +249,7 @@ struct rq_ctx {
     hipFunction_t mmq[RQ_NUM_FMTS + 1][3][3] = {};
     hipFunction_t mmqf[RQ_NUM_FMTS + 1][3] = {};
     hipFunction_t mmqd[RQ_NUM_FMTS][3][3] = {};
-    hipFunction_t mmqg[RQ_NUM_FMTS + 1][2][3] = {};  // 8 x G columns, G = 2, 4 (Q6_K and the mix: 2)
+    hipFunction_t mmqg[RQ_NUM_FMTS + 1][4][3] = {};  // 8 x G columns, G = 2, 4 (Q6_K also 6, 8; the mix: 2)
     // 16 x G columns with four-activation entries (Q4_0, Q8_0, Q4_K; G = 1,
     // 2, 4; sbw 2, 4), and the same classes of the fused gate/up (sbw 4)
     hipFunction_t mmqt[RQ_NUM_FMTS][3][2] = {};
@@ -679,13 +679,16 @@ bool mmq_has_t(int fmt, int S2) { return fmt != RQ_FMT_MIX_K && (S2 + 3) / 4 <= 
 // Q6_K runs the 16-column kernels for up to 16 columns only: holding its
 // weights for a second group makes them spill.
 int mmqt_max_cols(int fmt) { return fmt == RQ_FMT_Q6_K ? 16 : 64; }
-// (Q6_K, and so its mix with Q4_K, comes here with at most 16 columns:
-// use_cols.)
+// Q6_K takes up to 64 in its 8-column classes (8 x 6, 8 x 8 add each group's
+// k-parts as it ends, so LDS holds one group's partial sums next to 8 staged
+// columns of a 14336-wide row). (The mix comes here with at most 16 columns:
+// matvec_dispatch.)
 int mmq_max_cols(int fmt, int S2) {
-    return mmq_np(fmt, S2) > 1 ? 8 : fmt == RQ_FMT_Q6_K || fmt == RQ_FMT_MIX_K ? 16 : mmq_has_t(fmt, S2) ? 64 : 32;
+    if (mmq_np(fmt, S2) > 1) return 8;
+    return fmt == RQ_FMT_MIX_K ? 16 : mmq_has_t(fmt, S2) || fmt == RQ_FMT_Q6_K ? 64 : 32;
 }
 // Table index of an 8 x g class.
-int mmqg_index(int g) { return g == 2 ? 0 : 1; }
+int mmqg_index(int g) { return g == 2 ? 0 : g == 4 ? 1 : g == 6 ? 2 : 3; }
 // Group-count index of a 16-column class (g = 1, 2, 4).
 int mmqt_g_index(int g) { return g == 1 ? 0 : g == 2 ? 1 : 2; }
 // Super-blocks per wave of a 16-column launch: 4 for Q4_K; 2 for Q4_0 and
@@ -756,7 +759,8 @@ void mmq_layout(int fmt, int S2, bool dots, MmqPlan& L) {
     L.kxp = S2 * 256 + 64;  // 64 B of skew: columns start on different LDS banks
     L.pl_off = L.mp * L.kxp;
     L.part_off = L.pl_off + (mmq_planes(fmt) + (dots ? 1 : 0)) * L.mp * RQ_MMQ_NBP(S2) * 4;
-    L.lds = L.part_off + (dots ? 0 : L.ks * L.tr * 64 * (L.mp == 8 ? 2 : 1) * L.g * 4);  // every group's partial sums
+    // Partial sums of every group, or (g > 4) of one group at a time.
+    L.lds = L.part_off + (dots ? 0 : L.ks * L.tr * 64 * (L.mp == 8 ? 2 : 1) * (L.g > 4 ? 1 : L.g) * 4);
 }
 
 // A Q6_K vocabulary head (>= 16384 rows of 9 to 16 super-blocks) at one
@@ -884,7 +888,7 @@ MmqPlan mmq_cols(int fmt, int S2, int nc, bool allow16 = true) {
         return L;
     }
     L.mp = nc <= 1 ? 1 : nc <= 4 ? 4 : 8;
-    L.g = nc <= 8 ? 1 : nc <= 16 ? 2 : 4;
+    L.g = nc <= 8 ? 1 : nc <= 16 ? 2 : nc <= 32 || fmt != RQ_FMT_Q6_K ? 4 : nc <= 48 ? 6 : 8;
     return L;
 }
 
@@ -1049,11 +1053,10 @@ int cols_glu_groups(const rq_ctx* ctx, int fmt, int S) {
 //     (Q6_K 4096 x 14336 at 6 / 8: 20.1 / 32.0 against 20.1). At 8 columns
 //     4096-wide weights are mixed (Q4_K 4096 x 4096 9.3 / 7.3, Q6_K 14336 x
 //     4096 18.7 / 20.4).
-//   MFMA layout: Q6_K past 16 columns (1024 x 4096 at 32 / 64: 14.9 / 31.4
-//     us in its 8-column classes, 9.2 / 14.9 here; 14336 x 4096 at 32 28.0 /
-//     26.3), wide rows, which its 16-column class cannot stage, past 8 (4096
-//     x 14336 at 16 / 32 / 64: 22.0 / 37.9 / 72.9 -> 17.9 / 25.3 / 42.9 us;
-//     past 64 super-blocks every type, whose classes stop at 8 columns there);
+//   MFMA layout: Q6_K past 16 columns where q6_cols says, wide rows, which its
+//     16-column class cannot stage, past 8 (4096 x 14336 at 16 / 32 / 64: 22.0
+//     / 37.9 / 72.9 -> 17.9 / 25.3 / 42.9 us; past 64 super-blocks every type,
+//     whose classes stop at 8 columns there);
 //     the other types past 16 columns up to 512 tiles (Q4_K 4096 x 4096 at 32
 //     / 48 / 64: 10.9 / 17.8 / 19.0 -> 9.3 / 11.9 / 15.0 us; Q4_0 11.1 / 17.7
 //     / 19.0 -> 9.0 / 11.3 / 14.1), above which their classes read the
@@ -1061,6 +1064,21 @@ int cols_glu_groups(const rq_ctx* ctx, int fmt, int S) {
 //     against 22.4 us).
 // By the weight and m alone, so that a weight's result does not depend on
 // the weights beside it.
+//
+// q6_cols, Q6_K of up to 32 super-blocks in the MFMA layout past 16 columns: by
+// the rounds of one workgroup per CU that either takes, two tiles per
+// workgroup here, 16 waves' worth of k-parts there. A round here costs by its
+// steps of eight super-blocks, about half of one there up to 16 super-blocks
+// and two thirds from 17; below 9 a round there covers up to eight tiles per
+// workgroup at the same cost (us, there / here, at 17 columns: 1024 x 4096
+// 14.9 / 10.3, 8192 x 2048 14.4 / 10.9, 14336 x 4096 27.6 / 27.7, 14336 x 5120
+// 62 / 33, but 12288 x 4608 27.4 / 31.6, 20480 x 2304 25.6 / 32.6, 14336 x 512
+// 9.9 / 13.8, 32000 x 2048 28.3 / 35.6, 128256 x 1024 49 / 96).
+bool q6_cols(const rq_ctx* ctx, int64_t tiles, int S) {
+    const int64_t here = (tiles + 2 * ctx->cus - 1) / (2 * ctx->cus), tr = 16 / ((S + 3) / 4);
+    const int64_t there = (tiles + tr * ctx->cus - 1) / (tr * ctx->cus);
+    return S <= 8 ? here <= there : S <= 16 ? 2 * here <= 5 * there : 2 * here <= 3 * there;
+}
 bool use_cols(const rq_ctx* ctx, const rq_weight* w, int64_t m) {
     const int S = (int)((w->cols + 255) / 256);
     const bool mfma = use_mmq(w, m);
@@ -1070,7 +1088,7 @@ bool use_cols(const rq_ctx* ctx, const rq_weight* w, int64_t m) {
     else if (S > 64 || (S > 32 && w->fmt == RQ_FMT_Q6_K))
         use = m > 8;
     else
-        use = m > 16 && (w->fmt == RQ_FMT_Q6_K || w->tiles <= 512);
+        use = m > 16 && (w->fmt == RQ_FMT_Q6_K ? q6_cols(ctx, w->tiles, S) : w->tiles <= 512);
     return use && cols_plan(ctx, w->fmt, mfma, 1, S, m).rt > 0;
 }
 
@@ -1183,19 +1201,22 @@ rq_status cols_glu_launch(rq_ctx* ctx, const int8_t* xq, const uint16_t* xd, int
 }
 
 // One matvec group (one width and family) over Q8_1 activations: the weights
-// that run the column kernels in one launch, the others in another.
+// that run the column kernels in one launch, the others in another; the MFMA
+// layout's others past 16 columns, where Q4_K and Q6_K have no common class,
+// in one per type.
 rq_status matvec_dispatch(rq_ctx* ctx, const int8_t* xq, const uint16_t* xd, int64_t m, const rq_weight* const* ws,
                           float* const* outs, int count) {
-    const rq_weight* w[2][RQ_MV_TARGETS];
-    float* o[2][RQ_MV_TARGETS];
-    int n[2] = {0, 0};
+    const rq_weight* w[3][RQ_MV_TARGETS];
+    float* o[3][RQ_MV_TARGETS];
+    int n[3] = {0, 0, 0};
     for (int i = 0; i < count; i++) {
-        const int c = use_cols(ctx, ws[i], m) ? 1 : 0;
+        const int c = use_cols(ctx, ws[i], m) ? 1 : m > 16 && use_mmq(ws[i], m) && ws[i]->fmt == RQ_FMT_Q6_K ? 2 : 0;
         w[c][n[c]] = ws[i];
         o[c][n[c]++] = outs[i];
     }
     rq_status st = RQ_OK;
     if (n[1] > 0) st = cols_launch(ctx, xq, xd, m, w[1], o[1], n[1]);
+    if (st == RQ_OK && n[2] > 0) st = mmq_launch(ctx, xq, xd, nullptr, m, w[2], (void* const*)o[2], n[2], false);
     if (st != RQ_OK || n[0] == 0) return st;
     if (use_mmq(w[0][0], m)) return mmq_launch(ctx, xq, xd, nullptr, m, w[0], (void* const*)o[0], n[0], false);
     return matvec_launch(ctx, xq, xd, nullptr, m, w[0], o[0], n[0]);
@@ -1516,7 +1537,8 @@ extern "C" rq_status rq_open(int device, rq_ctx** out) {
             if (kMmqSbw[si] > mmq_sbw_max(f)) continue;
             snprintf(name, sizeof name, "rq_mmqf_%s_%d", kFmtSuffix[f], kMmqSbw[si]);
             st = getm(ctx->mmq_mod, &ctx->mmqf[f][si], name);
-            for (int gi = 0; gi < (f == RQ_FMT_Q6_K ? 1 : 2) && st == RQ_OK; gi++) {
+            for (int gi = 0; gi < 4 && st == RQ_OK; gi++) {
+                if (gi >= 2 && (f != RQ_FMT_Q6_K || kMmqSbw[si] != 4)) continue;  // 8 x 6, 8 x 8: Q6_K only
                 snprintf(name, sizeof name, "rq_mmq_%s_8x%d_%d", kFmtSuffix[f], 2 * (gi + 1), kMmqSbw[si]);
                 st = getm(ctx->mmq_mod, &ctx->mmqg[f][gi][si], name);
             }

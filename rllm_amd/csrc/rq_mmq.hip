@@ -374,6 +374,33 @@ __device__ __forceinline__ void mmq_reduce(const RqMmqParams& P, const RqMmqTarg
     }
 }
 
+// Classes of more column groups than the LDS holds partial sums for (Q6_K 8 x
+// 6, 8 x 8: up to 64 columns over 14336-wide rows, whose staging of 8 columns
+// alone takes 115 KB) add each group's k-parts as soon as the group is done:
+// one partial slot per wave, reused by the next group after its staging
+// barrier. The sums and their order are mmq_reduce's.
+template <int G>
+struct GroupReduce {
+    static constexpr bool on = G > 4;
+};
+
+template <int MP, int NACC>
+__device__ __forceinline__ void mmq_reduce_group(const RqMmqParams& P, const RqMmqTarget& T, int gi) {
+    const int threads = blockDim.x, tid = threadIdx.x;
+    const int blk = blockIdx.x, ks = P.ks;
+    const float* part = (const float*)(mmq_lds + P.part_off);
+    __syncthreads();
+    float* out = (float*)T.out;
+    for (int it = tid; it < P.tr * MP * 16; it += threads) {
+        const int tl2 = it / (MP * 16), a = (it >> 4) % MP, nn = it & 15, ag = gi * MP + a;
+        const int tile2 = (blk - T.wg_start) * P.tr + tl2, row = tile2 * 16 + nn;
+        if (ag >= P.m || tile2 >= T.tiles || row >= T.n) continue;
+        float s = 0.f;
+        for (int q = 0; q < ks; q++) s += part_at<MP>(part, tl2 * ks + q, a, nn);
+        gmem(out)[(int64_t)ag * T.n + row] = s;
+    }
+}
+
 // rq_mmqglu_*: the workgroup's two tiles of gate (waves 0 .. ks tr - 1) and
 // of up (the next ks tr) meet as h = act(g) * u (act_apply, as rq_act_mul),
 // written as f32 (hf, when set) and, per column, as the Q8_1 block of the 32
@@ -505,7 +532,7 @@ __device__ __forceinline__ void mmq_body(const RqMmqParams& P) {
     // 18.6; at one column the MFMA decode step 1138 -> 1111 us). Chosen at
     // compile time: a run-time choice slowed the launches that did not take
     // it.
-    constexpr bool PIPE = !WIDE;
+    constexpr bool PIPE = !WIDE && G <= 4;
     if constexpr (PIPE)
         load_h(0);
     else
@@ -1229,11 +1256,13 @@ __device__ __forceinline__ void mmq6_body(const RqMmqParams& P) {
     // no arithmetic overlapping it (4096 x 14336 at 4 / 8 / 16 / 32 columns:
     // 12.8 / 15.8 / 24.0 / 39.6 -> 11.4 / 13.7 / 21.7 / 37.6 us; the
     // 128256 x 4096 head at 8 columns 72.8 -> 69.3, at 4 62.0 -> 63.3). Not
-    // for one f32 column (the decode step on f32 inputs 1184 -> 1203 us). Chosen at compile time (a run-time
+    // in the 8 x 6 / 8 x 8 classes, whose weights spill (48 / 64 columns
+    // 55.7 / 72.3 -> 57.3 / 74.0 us), nor for one f32 column (the decode
+    // step on f32 inputs 1184 -> 1203 us). Chosen at compile time (a run-time
     // choice slowed the launches that did not take it). The direct column
     // (DX) has no staging and the wide kernels walk the row in passes: they
     // load everything at once.
-    constexpr bool PIPE = MP > 1 && !DX && !WIDE;
+    constexpr bool PIPE = MP > 1 && !DX && !WIDE && G <= 4;
     if constexpr (PIPE) {
         load_d();
         load_sb(0);
@@ -1382,11 +1411,16 @@ __device__ __forceinline__ void mmq6_body(const RqMmqParams& P) {
     if (!DOTS) {
 #pragma unroll
         for (int e = 0; e < NACC; e++) y[e] *= 0.25f;
-        mmq_part_store<MP, NACC>(P, y, wave * G + gi, lane);
+        if (GroupReduce<G>::on) {
+            mmq_part_store<MP, NACC>(P, y, wave, lane);
+            mmq_reduce_group<MP, NACC>(P, T, gi);
+        } else {
+            mmq_part_store<MP, NACC>(P, y, wave * G + gi, lane);
+        }
     }
     }  // column groups
     tl_mark(tlm, 4);
-    if (DOTS) {
+    if (DOTS || GroupReduce<G>::on) {
         tl_store(tlm);
         return;
     }
@@ -1576,23 +1610,20 @@ __device__ __forceinline__ void mmq_run(const RqMmqParams& P) {
     RQ_MMQ(NAME, FMT, 4, SBW)                                                                    \
     RQ_MMQ(NAME, FMT, 8, SBW)                                                                    \
     RQ_MMQ_G(NAME, FMT, 2, SBW)                                                                  \
+    RQ_MMQ_G(NAME, FMT, 4, SBW)                                                                  \
     extern "C" __global__ __launch_bounds__(1024) void rq_mmqf_##NAME##_##SBW(RqMmqParams p) {     \
         mmq_run<FMT, 1, SBW, true, false>(p);                                                    \
     }
 
 // Q8_0 holds 16 B of codes per lane per window: sbw = 8 would need 128 registers of them.
-// (8 x 4: the formats whose 17 to 32 columns can run here; Q6_K's go to rq_cols_*.)
-#define RQ_MMQ_SET4(NAME, FMT, SBW) \
-    RQ_MMQ_SET(NAME, FMT, SBW)      \
-    RQ_MMQ_G(NAME, FMT, 4, SBW)
-RQ_MMQ_SET4(q4_0, RQ_FMT_Q4_0, 2)
-RQ_MMQ_SET4(q4_0, RQ_FMT_Q4_0, 4)
-RQ_MMQ_SET4(q4_0, RQ_FMT_Q4_0, 8)
-RQ_MMQ_SET4(q8_0, RQ_FMT_Q8_0, 2)
-RQ_MMQ_SET4(q8_0, RQ_FMT_Q8_0, 4)
-RQ_MMQ_SET4(q4_k, RQ_FMT_Q4_K, 2)
-RQ_MMQ_SET4(q4_k, RQ_FMT_Q4_K, 4)
-RQ_MMQ_SET4(q4_k, RQ_FMT_Q4_K, 8)
+RQ_MMQ_SET(q4_0, RQ_FMT_Q4_0, 2)
+RQ_MMQ_SET(q4_0, RQ_FMT_Q4_0, 4)
+RQ_MMQ_SET(q4_0, RQ_FMT_Q4_0, 8)
+RQ_MMQ_SET(q8_0, RQ_FMT_Q8_0, 2)
+RQ_MMQ_SET(q8_0, RQ_FMT_Q8_0, 4)
+RQ_MMQ_SET(q4_k, RQ_FMT_Q4_K, 2)
+RQ_MMQ_SET(q4_k, RQ_FMT_Q4_K, 4)
+RQ_MMQ_SET(q4_k, RQ_FMT_Q4_K, 8)
 // Q6_K holds 48 B of codes per lane per super-block: sbw = 8 would need 96 registers of them.
 RQ_MMQ_SET(q6_k, RQ_FMT_Q6_K, 2)
 RQ_MMQ_SET(q6_k, RQ_FMT_Q6_K, 4)
@@ -1604,6 +1635,8 @@ extern "C" __global__ __launch_bounds__(512) void rq_mmq_q6_k_1_8(RqMmqParams p)
 extern "C" __global__ __launch_bounds__(512) void rq_mmqf_q6_k_8(RqMmqParams p) {
     mmq_run<RQ_FMT_Q6_K, 1, 8, true, false>(p);
 }
+RQ_MMQ_G(q6_k, RQ_FMT_Q6_K, 6, 4)
+RQ_MMQ_G(q6_k, RQ_FMT_Q6_K, 8, 4)
 // Fused gate/up + activation + Q8_1 of the product (the reference's
 // mmq_glu_*), 4 super-blocks per wave (rows of up to 16: the two weights'
 // k-parts of two tiles fill at most 16 waves); one column over rows of 9 to

@@ -115,3 +115,29 @@ def test_cols_gated_ffn(gpu, orc, tname, f, d, m):
     want = gpu.alloc(m * 256)
     gpu.matvec(gpu.quantize_q8_1(h, m, f), down, want, m)
     assert torch.equal(out.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("n,k", [(9216, 512), (16400, 512), (8208, 1024), (20480, 2304), (8208, 4352), (8240, 2048)])
+@pytest.mark.parametrize("m", [17, 33, 48, 49, 64])
+def test_q6_k_rows_that_keep_the_int8_classes(gpu, orc, n, k, m):
+    """MFMA-layout Q6_K where the int8 classes take fewer rounds (short rows
+    of more than 512 tiles, and where three or five tiles fit a workgroup):
+    columns as in an 8-column launch, bit for bit, and within 1e-3 of the
+    oracle."""
+    t = TYPES["Q6_K"]
+    w = orc.random_weight(90, t, n, k)
+    gpu.set_kernels("mfma")
+    wg = upload(gpu, t, w, n, k)
+    gpu.set_kernels("auto")
+    qs, d, s = _q8(orc, 91 + m, m, k)
+    out, eight = gpu.alloc(m * n), gpu.alloc(8 * n)
+    gpu.matvec(q8_1_to_device(gpu, qs, d, s), wg, out, m)
+    for c0 in (0, 8, m - 8):
+        part = q8_1_to_device(gpu, qs[c0 * k:(c0 + 8) * k], d[c0 * k // 32:(c0 + 8) * k // 32], s[c0 * k // 32:(c0 + 8) * k // 32])
+        gpu.matvec(part, wg, eight, 8)
+        assert torch.equal(out[c0 * n:(c0 + 8) * n], eight[:8 * n]), f"columns {c0}.."
+    rows = np.r_[0:17, n - 17:n]
+    rb = w.reshape(n, -1)
+    want = orc.matvec_q8_1(t, np.ascontiguousarray(rb[rows]).reshape(-1), len(rows), k, qs, d, m)
+    got = gpu.to_host(out, m * n).reshape(m, n)[:, rows].reshape(-1)
+    orc.assert_close(f"Q6_K {n}x{k} m={m}", want, got, 1e-3)
