@@ -1002,37 +1002,74 @@ int cols_lds_bytes(int fmt, bool mfma, int rt, int cg, int S) {
     return std::max(stage + x, RQ_COLS_PARTS * rt * cg * 1024);
 }
 
-// Most tiles per workgroup there is a kernel for (more would spill).
+// Most tiles per workgroup there is a kernel for (more would spill far: of
+// these the 2 x 3 ones of the MFMA layout and the 4 x 2 ones of Q8_0 and Q6_K
+// spill up to 24 registers, which their times below hold).
 int cols_max_rt(bool mfma, int cg) { return cg <= 2 ? (mfma ? 2 : 4) : cg == 3 ? 2 : 1; }
 
+// Microseconds of a step (eight super-blocks of the row) in the first and in
+// each further round of workgroups, by layout (dot4, MFMA), type (Q4, Q8_0,
+// Q6_K), column groups and log2 of the tiles per workgroup (0: no kernel).
+const float kColsStep[2][3][RQ_COLS_MAX_GROUPS][3][2] = {
+    {{{{2.1f, 1.3f}, {3.2f, 2.0f}, {5.4f, 6.0f}},
+      {{3.3f, 3.3f}, {4.5f, 4.7f}, {7.0f, 7.8f}},
+      {{4.6f, 4.7f}, {6.1f, 6.3f}},
+      {{5.9f, 6.0f}}},
+     {{{2.4f, 1.6f}, {3.8f, 4.3f}, {6.5f, 7.8f}},
+      {{3.4f, 3.5f}, {5.1f, 5.5f}, {9.5f, 10.5f}},
+      {{4.6f, 4.9f}, {6.7f, 7.0f}},
+      {{6.0f, 6.3f}}},
+     {{{2.6f, 1.6f}, {4.4f, 4.3f}, {7.5f, 8.1f}},
+      {{3.8f, 3.7f}, {5.6f, 5.8f}, {9.5f, 10.5f}},
+      {{5.0f, 5.2f}, {7.2f, 7.4f}},
+      {{6.3f, 6.3f}}}},
+    {{{{1.7f, 1.2f}, {2.7f, 2.6f}},
+      {{3.1f, 2.8f}, {4.1f, 4.1f}},
+      {{4.2f, 4.1f}, {5.6f, 5.5f}},
+      {{5.4f, 5.3f}}},
+     {{{1.8f, 1.3f}, {2.9f, 3.0f}},
+      {{3.2f, 2.9f}, {4.5f, 4.5f}},
+      {{4.3f, 4.1f}, {8.8f, 8.2f}},
+      {{5.4f, 5.3f}}},
+     {{{2.1f, 1.5f}, {3.4f, 3.7f}},
+      {{3.5f, 3.3f}, {4.9f, 4.8f}},
+      {{4.6f, 4.3f}, {7.9f, 7.3f}},
+      {{6.0f, 5.7f}}}}};
+
 // Launches of m columns over `tiles` 16-row tiles: rt tiles per workgroup and
-// cg column groups per launch, rt = 0 where nothing fits the LDS.
-//   rt: tiles of a workgroup share its reads and conversion of the
-//       activations, but a launch wants a workgroup for every CU. Q4_K, dot4
-//       layout at 16 columns, 1 / 2 / 4 tiles: 4096 x 4096 (256 tiles) 7.4 /
-//       9.0 / 13.6 us, 14336 x 4096 (896 tiles) 17.0 / 16.5 / 13.9 us.
-//   cg: 64 columns in one launch hold one tile per workgroup (15.3 us for
-//       4096 x 4096), so weights that want two or more go as two launches of
-//       32 (14336 x 4096: 56.3 us in one launch, 18.7 in each of two).
+// cg column groups per launch, rt = 0 where nothing fits the LDS. Tiles of a
+// workgroup share its reads and conversion of the activations, but a round
+// holds one workgroup per CU (two one-tile ones of one column group), so
+// whether more of them or fewer columns per launch pay depends on the rounds:
+// the choice with the lowest estimated time, 3.2 us a launch, kColsStep per
+// step and 1 us per further round. (By tiles alone, two from 385 and four from
+// 768, 257 to 384 tiles took two rounds of one each: Q4_K 6144 x 4096, MFMA
+// layout, at 17 / 64 columns 17.6 / 28.9 us against 13.4 / 24.6 at two; Q8_0
+// 14336 x 4096, dot4, at 24 45 us at four against 28.) Measured over 15 sizes
+// from 96 to 128256 rows, 512 to 14336 columns and 9 to 64 tokens (13404
+// calls): the choice is within 5 % of the best in 97 %, within 14 % in all.
 struct ColsPlan {
     int rt = 0, cg = 0;
     int64_t launches = 0;
 };
 ColsPlan cols_plan(const rq_ctx* ctx, int fmt, bool mfma, int64_t tiles, int S, int64_t m) {
-    ColsPlan p;
-    const bool many = tiles > ctx->cus * 3 / 2;
-    for (int max_cg = many ? 3 : RQ_COLS_MAX_GROUPS; max_cg >= 1; max_cg--) {
+    ColsPlan best;
+    double best_us = 0;
+    const int type = fmt == RQ_FMT_Q8_0 ? 1 : fmt == RQ_FMT_Q6_K || fmt == RQ_FMT_MIX_K ? 2 : 0, steps = (S + 7) / 8;
+    for (int max_cg = RQ_COLS_MAX_GROUPS; max_cg >= 1; max_cg--) {
         const int64_t per = RQ_COLS_GROUP * max_cg;
+        ColsPlan p;
         p.launches = (m + per - 1) / per;
         p.cg = (int)(((m + p.launches - 1) / p.launches + RQ_COLS_GROUP - 1) / RQ_COLS_GROUP);
-        int rt = std::min(cols_max_rt(mfma, p.cg), tiles >= 3 * ctx->cus ? 4 : many ? 2 : 1);
-        for (; rt >= 1; rt /= 2)
-            if (cols_lds_bytes(fmt, mfma, rt, p.cg, S) <= ctx->lds_wide) {
-                p.rt = rt;
-                return p;
-            }
+        for (p.rt = 1; p.rt <= cols_max_rt(mfma, p.cg); p.rt *= 2) {
+            if (cols_lds_bytes(fmt, mfma, p.rt, p.cg, S) > ctx->lds_wide) break;
+            const float* step = kColsStep[mfma ? 1 : 0][type][p.cg - 1][p.rt >> 1];
+            const int64_t wgs = (tiles + p.rt - 1) / p.rt, rounds = (wgs + ctx->cus - 1) / ctx->cus;
+            const double us = p.launches * (3.2 + step[0] * steps + (rounds - 1) * (1.0 + step[1] * steps));
+            if (best.rt == 0 || us < best_us) best = p, best_us = us;
+        }
     }
-    return p;
+    return best;
 }
 
 // The fused gate/up launches (dot4 layout): two tiles of each weight per

@@ -141,3 +141,60 @@ def test_q6_k_rows_that_keep_the_int8_classes(gpu, orc, n, k, m):
     want = orc.matvec_q8_1(t, np.ascontiguousarray(rb[rows]).reshape(-1), len(rows), k, qs, d, m)
     got = gpu.to_host(out, m * n).reshape(m, n)[:, rows].reshape(-1)
     orc.assert_close(f"Q6_K {n}x{k} m={m}", want, got, 1e-3)
+
+
+# Rows for two and for four tiles per workgroup (cols_plan: more tiles than
+# CUs, and twice as many), the last tile partly past the rows.
+@pytest.mark.parametrize("tname", list(TYPES))
+@pytest.mark.parametrize("family,n,k", [("dot4", 6396, 768), ("dot4", 12792, 512), ("dot4", 12810, 1280),
+                                        ("mfma", 6396, 768), ("mfma", 8182, 2304)])
+def test_cols_several_tiles_per_workgroup(gpu, orc, tname, family, n, k):
+    """Columns in every group count, single launches and two: within the
+    bound of the oracle on the first and last rows, and bit-identical to a
+    weight that holds these rows alone (one tile per workgroup)."""
+    t = TYPES[tname]
+    w = orc.random_weight(95, t, n, k)
+    rb = w.reshape(n, -1)
+    rows = np.r_[0:33, n - 43:n]
+    few = np.ascontiguousarray(rb[rows]).reshape(-1)
+    gpu.set_kernels(family)
+    wg, fg = upload(gpu, t, w, n, k), upload(gpu, t, few, len(rows), k)
+    gpu.set_kernels("auto")
+    for m in (9, 20, 33, 48, 64, 70):
+        if family == "mfma" and m <= 16:
+            continue
+        qs, d, s = _q8(orc, 96 + m, m, k)
+        xq = q8_1_to_device(gpu, qs, d, s)
+        out, part = gpu.alloc(m * n + 8), gpu.alloc(m * len(rows))
+        out.fill_(float("nan"))
+        gpu.matvec(xq, wg, out, m)
+        gpu.matvec(xq, fg, part, m)
+        got = gpu.to_host(out)
+        assert np.isnan(got[m * n:]).all(), "wrote past the output"
+        got = np.ascontiguousarray(got[:m * n].reshape(m, n)[:, rows]).reshape(-1)
+        assert np.isfinite(got).all()
+        orc.assert_close(f"{tname} {n}x{k} m={m} {family}", orc.matvec_q8_1(t, few, len(rows), k, qs, d, m), got, TOL)
+        assert np.array_equal(got.view(np.uint32), gpu.to_host(part, m * len(rows)).view(np.uint32)), f"m={m}"
+
+
+@pytest.mark.parametrize("family", ["dot4", "mfma"])
+@pytest.mark.parametrize("rows", [(4100, 1030, 1100), (6400, 3200, 3300)])
+def test_cols_mixed_launch_of_several_tiles(gpu, orc, family, rows):
+    """Q4_K and Q6_K in one launch of more tiles than CUs, and than twice as
+    many: each output as in its weight's own launch."""
+    k, m = 1280, 40
+    spec = list(zip((12, 14, 12), rows))
+    gpu.set_kernels(family)
+    wgs = [upload(gpu, t, orc.random_weight(97 + i, t, n, k), n, k) for i, (t, n) in enumerate(spec)]
+    gpu.set_kernels("auto")
+    for cols in (9, 17, m, 70):
+        x = _q8(orc, 98 + cols, cols, k)
+        xq = q8_1_to_device(gpu, *x)
+        outs = [gpu.alloc(cols * n) for n in rows]
+        gpu.matvec_many(xq, wgs, outs, cols)
+        if family == "mfma" and cols <= 16:
+            continue  # (the mixed int8 class there)
+        for n, wg, out in zip(rows, wgs, outs):
+            own = gpu.alloc(cols * n)
+            gpu.matvec(xq, wg, own, cols)
+            assert torch.equal(own, out), f"{n} rows, {cols} columns"
