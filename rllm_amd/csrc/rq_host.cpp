@@ -1092,15 +1092,26 @@ int cols_glu_groups(const rq_ctx* ctx, int fmt, int S) {
 //     4096 18.7 / 20.4).
 //   MFMA layout: Q6_K past 16 columns where q6_cols says, wide rows, which its
 //     16-column class cannot stage, past 8 (4096 x 14336 at 16 / 32 / 64: 22.0
-//     / 37.9 / 72.9 -> 17.9 / 25.3 / 42.9 us; past 64 super-blocks every type,
-//     whose classes stop at 8 columns there);
-//     the other types past 16 columns up to 512 tiles (Q4_K 4096 x 4096 at 32
-//     / 48 / 64: 10.9 / 17.8 / 19.0 -> 9.3 / 11.9 / 15.0 us; Q4_0 11.1 / 17.7
-//     / 19.0 -> 9.0 / 11.3 / 14.1), above which their classes read the
-//     activations for four tiles at once (Q4_K 14336 x 4096 at 32: 18.9
-//     against 22.4 us).
-// By the weight and m alone, so that a weight's result does not depend on
-// the weights beside it.
+//     / 37.9 / 72.9 -> 17.9 / 25.3 / 42.9 us), but below 40 super-blocks on no
+//     more tiles than CUs past 16 (4096 x 8448 at 9 / 16 12.2 / 13.4 in the
+//     classes, 14.3 / 13.8 here); past 64 super-blocks every type, whose
+//     classes stop at 8 columns there;
+//     the other types past 16 columns: from 17 super-blocks, where one tile's
+//     k-parts leave no room for a second in a workgroup of theirs (us, classes
+//     / here, at 17 and 64 columns: Q4_K 4096 x 5120 13.7 / 12.3 and 25.1 /
+//     19.0, 14336 x 5120 33.8 / 28.5 and 64 / 53, Q8_0 28672 x 6144 87 / 66 and
+//     175 / 126), of shorter rows up to two tiles per CU (Q4_K 4096 x 4096 at
+//     32 / 48 / 64: 10.9 / 17.8 / 19.0 -> 9.3 / 11.9 / 15.0 us), above which
+//     the classes read the activations for four tiles at once (14336 x 4096
+//     at 32: 18.9 against 22.4 us). Past 48 columns two tiles per workgroup
+//     take two launches here, which cost the classes' four-fold staging of
+//     Q8_0's rows up to 9 super-blocks, and of the others' from 13 (Q8_0 8192
+//     x 1024 at 64 14.6 / 16.8, Q4_K 8192 x 4096 22.9 / 25.2; between, Q4_K
+//     8192 x 3072 26.2 / 22.0).
+// By the weight and m alone, so that a weight's result does not depend on the
+// weights beside it: a group of MFMA-layout weights on both sides runs as two
+// launches (Q4_K 9216 + 2 x 2304 rows of 4096 at 17 columns 30 us, 19.5 when
+// all ran the classes).
 //
 // q6_cols, Q6_K of up to 32 super-blocks in the MFMA layout past 16 columns: by
 // the rounds of one workgroup per CU that either takes, two tiles per
@@ -1110,11 +1121,13 @@ int cols_glu_groups(const rq_ctx* ctx, int fmt, int S) {
 // workgroup at the same cost (us, there / here, at 17 columns: 1024 x 4096
 // 14.9 / 10.3, 8192 x 2048 14.4 / 10.9, 14336 x 4096 27.6 / 27.7, 14336 x 5120
 // 62 / 33, but 12288 x 4608 27.4 / 31.6, 20480 x 2304 25.6 / 32.6, 14336 x 512
-// 9.9 / 13.8, 32000 x 2048 28.3 / 35.6, 128256 x 1024 49 / 96).
-bool q6_cols(const rq_ctx* ctx, int64_t tiles, int S) {
+// 9.9 / 13.8, 32000 x 2048 28.3 / 35.6, 128256 x 1024 49 / 96), from four
+// super-blocks on at a little more in the class of 33 to 48 columns (9216 x
+// 2048: 26.0 / 23.1).
+bool q6_cols(const rq_ctx* ctx, int64_t tiles, int S, int64_t m) {
     const int64_t here = (tiles + 2 * ctx->cus - 1) / (2 * ctx->cus), tr = 16 / ((S + 3) / 4);
     const int64_t there = (tiles + tr * ctx->cus - 1) / (tr * ctx->cus);
-    return S <= 8 ? here <= there : S <= 16 ? 2 * here <= 5 * there : 2 * here <= 3 * there;
+    return S <= 8 ? here <= there * (S >= 4 && m > 32 && m <= 48 ? 2 : 1) : S <= 16 ? 2 * here <= 5 * there : 2 * here <= 3 * there;
 }
 bool use_cols(const rq_ctx* ctx, const rq_weight* w, int64_t m) {
     const int S = (int)((w->cols + 255) / 256);
@@ -1123,9 +1136,12 @@ bool use_cols(const rq_ctx* ctx, const rq_weight* w, int64_t m) {
     if (!mfma)
         use = m >= (S > 32 ? 7 : 9);
     else if (S > 64 || (S > 32 && w->fmt == RQ_FMT_Q6_K))
-        use = m > 8;
+        use = m > (S >= 40 || w->tiles > ctx->cus ? 8 : 16);
+    else if (w->fmt == RQ_FMT_Q6_K)
+        use = m > 16 && q6_cols(ctx, w->tiles, S, m);
     else
-        use = m > 16 && (w->fmt == RQ_FMT_Q6_K ? q6_cols(ctx, w->tiles, S) : w->tiles <= 512);
+        use = m > 16 && (S > 16 || (w->tiles <= 2 * ctx->cus && (m <= 48 || w->tiles <= ctx->cus ||
+                                                                (w->fmt == RQ_FMT_Q8_0 ? S > 9 : S <= 12))));
     return use && cols_plan(ctx, w->fmt, mfma, 1, S, m).rt > 0;
 }
 
