@@ -1086,10 +1086,13 @@ int cols_glu_groups(const rq_ctx* ctx, int fmt, int S) {
 //     64 columns: Q4_K 4096 x 4096 17.5 / 7.3 and 69.7 / 15.6, 14336 x 4096
 //     36.7 / 13.7 and 144 / 37.5; Q8_0 11008 x 4096 30.5 / 17.4 and 120 / 44;
 //     Q6_K 4096 x 14336 65 / 20 and 180 / 43, 128256 x 4096 227 / 144 and 894
-//     / 390); rows of more than 32 super-blocks, one to a tile there, from 7
-//     (Q6_K 4096 x 14336 at 6 / 8: 20.1 / 32.0 against 20.1). At 8 columns
-//     4096-wide weights are mixed (Q4_K 4096 x 4096 9.3 / 7.3, Q6_K 14336 x
-//     4096 18.7 / 20.4).
+//     / 390), but up to two super-blocks on many tiles, of which a round here
+//     uses two of eight waves, at no count (us at 16: Q4_K 65536 x 512 22 / 21,
+//     128256 x 512 32 / 40; Q6_K 28672 x 512 16 / 16, at 10 13.4 / 15.8) and up
+//     to four on the largest not to 12 (128256 x 1024 at 9 37 / 41, at 16 53 /
+//     44). At 8 columns 4096-wide weights are mixed (Q4_K 4096 x 4096 9.3 /
+//     7.3, Q6_K 14336 x 4096 18.7 / 20.4).
+//     Rows of more than 32 super-blocks, one to a tile there: cols_from_wide.
 //   MFMA layout: Q6_K past 16 columns where q6_cols says, wide rows, which its
 //     16-column class cannot stage, past 8 (4096 x 14336 at 16 / 32 / 64: 22.0
 //     / 37.9 / 72.9 -> 17.9 / 25.3 / 42.9 us), but below 40 super-blocks on no
@@ -1129,19 +1132,37 @@ bool q6_cols(const rq_ctx* ctx, int64_t tiles, int S, int64_t m) {
     const int64_t there = (tiles + tr * ctx->cus - 1) / (tr * ctx->cus);
     return S <= 8 ? here <= there * (S >= 4 && m > 32 && m <= 48 ? 2 : 1) : S <= 16 ? 2 * here <= 5 * there : 2 * here <= 3 * there;
 }
+//
+// cols_from_wide, the columns from which rows of S > 32 super-blocks in the
+// dot4 layout come here: 7 where the launch fills the CUs (us, dot4 / here, at
+// 7 and 8: Q4_K 4096 x 14336 21.9 / 20.1 and 28.7 / 19.9, Q6_K 8192 x 14336 44
+// / 40 and 61 / 38, Q8_0 27 / 22.5 and 39 / 22.5); on fewer tiles one round
+// here costs what it costs and the dot4 launch less (1024 x 11008: Q8_0 at 7 /
+// 8 / 9 11.3 / 12.0 / 16.6 against 18.6, Q6_K at 7 / 8 16.3 / 18.1 against
+// 18.6), Q4's excepted up to 64 super-blocks (16.6 / 18.4 against 15.4).
+int64_t cols_from_wide(const rq_ctx* ctx, const rq_weight* w, int S) {
+    const bool full = w->rows >= 16 * ctx->cus;
+    if (w->fmt == RQ_FMT_Q8_0) return full ? 7 : 10;
+    if (w->fmt == RQ_FMT_Q6_K) return w->rows > 16 * ctx->cus ? 7 : S <= 64 ? 8 : 9;
+    return full || S <= 64 ? 7 : 9;
+}
 bool use_cols(const rq_ctx* ctx, const rq_weight* w, int64_t m) {
     const int S = (int)((w->cols + 255) / 256);
     const bool mfma = use_mmq(w, m);
     bool use;
-    if (!mfma)
-        use = m >= (S > 32 ? 7 : 9);
+    const int64_t tiles = (w->rows + 15) / 16;
+    const bool q4 = w->fmt == RQ_FMT_Q4_K || w->fmt == RQ_FMT_Q4_0;
+    if (!mfma && S > 32)
+        use = m >= cols_from_wide(ctx, w, S);
+    else if (!mfma)
+        use = m > 8 && !(S <= 2 && tiles > (q4 ? 7 : 5) * ctx->cus) && !(S <= 4 && tiles > 16 * ctx->cus && m <= 12);
     else if (S > 64 || (S > 32 && w->fmt == RQ_FMT_Q6_K))
-        use = m > (S >= 40 || w->tiles > ctx->cus ? 8 : 16);
+        use = m > (S >= 40 || tiles > ctx->cus ? 8 : 16);
     else if (w->fmt == RQ_FMT_Q6_K)
-        use = m > 16 && q6_cols(ctx, w->tiles, S, m);
+        use = m > 16 && q6_cols(ctx, tiles, S, m);
     else
-        use = m > 16 && (S > 16 || (w->tiles <= 2 * ctx->cus && (m <= 48 || w->tiles <= ctx->cus ||
-                                                                (w->fmt == RQ_FMT_Q8_0 ? S > 9 : S <= 12))));
+        use = m > 16 && (S > 16 || (tiles <= 2 * ctx->cus &&
+                                    (m <= 48 || tiles <= ctx->cus || (w->fmt == RQ_FMT_Q8_0 ? S > 9 : S <= 12))));
     return use && cols_plan(ctx, w->fmt, mfma, 1, S, m).rt > 0;
 }
 

@@ -216,3 +216,20 @@ def test_rows_that_keep_the_16_column_classes(gpu, orc, tname, n, k, m):
     gpu.matvec(q8_1_to_device(gpu, qs, d, s), wg, out, m)
     gpu.matvec(q8_1_to_device(gpu, qs[:16 * k], d[:16 * k // 32], s[:16 * k // 32]), wg, part, 16)
     assert torch.equal(out[:16 * n], part)
+
+
+@pytest.mark.parametrize("tname,n,k,m", [("Q8_0", 96, 11008, 7), ("Q8_0", 2040, 14336, 9), ("Q6_K", 1024, 11008, 7),
+                                         ("Q4_K", 96, 20480, 8), ("Q4_0", 65536, 512, 12), ("Q6_K", 28672, 512, 16),
+                                         ("Q8_0", 65600, 1024, 12)])
+def test_rows_that_keep_the_dot4_kernels(gpu, orc, tname, n, k, m):
+    """Default layout: wide rows on fewer tiles than CUs at 7 to 9 columns, and
+    many short rows: columns as in one-column calls, bit for bit."""
+    t = TYPES[tname]
+    wg = upload(gpu, t, orc.random_weight(94, t, n, k), n, k)
+    qs, d, s = _q8(orc, 95 + m, m, k)
+    out, one = gpu.alloc(m * n), gpu.alloc(n)
+    gpu.matvec(q8_1_to_device(gpu, qs, d, s), wg, out, m)
+    for c in (0, m - 1):
+        gpu.matvec(q8_1_to_device(gpu, qs[c * k:(c + 1) * k], d[c * k // 32:(c + 1) * k // 32],
+                                  s[c * k // 32:(c + 1) * k // 32]), wg, one, 1)
+        assert torch.equal(out[c * n:(c + 1) * n], one), f"column {c}"
