@@ -1080,18 +1080,61 @@ int cols_glu_groups(const rq_ctx* ctx, int fmt, int S) {
     return cg;
 }
 
+// q6_cols, Q6_K of up to 32 super-blocks in the MFMA layout past 16 columns: by
+// the rounds of one workgroup per CU that either takes, two tiles per
+// workgroup here, 16 waves' worth of k-parts there. A round here costs by its
+// steps of eight super-blocks, about half of one there up to 16 super-blocks
+// and two thirds from 17; below 9 a round there covers up to eight tiles per
+// workgroup at the same cost (us, there / here, at 17 columns: 1024 x 4096
+// 14.9 / 10.3, 8192 x 2048 14.4 / 10.9, 14336 x 4096 27.6 / 27.7, 14336 x 5120
+// 62 / 33, but 12288 x 4608 27.4 / 31.6, 20480 x 2304 25.6 / 32.6, 14336 x 512
+// 9.9 / 13.8, 32000 x 2048 28.3 / 35.6, 128256 x 1024 49 / 96), from four
+// super-blocks on at a little more in the class of 33 to 48 columns (9216 x
+// 2048: 26.0 / 23.1).
+bool q6_cols(const rq_ctx* ctx, int64_t tiles, int S, int64_t m) {
+    const int64_t here = (tiles + 2 * ctx->cus - 1) / (2 * ctx->cus), tr = 16 / ((S + 3) / 4);
+    const int64_t there = (tiles + tr * ctx->cus - 1) / (tr * ctx->cus);
+    if (S <= 8) return here <= there * (S >= 4 && m > 32 && m <= 48 ? 2 : 1);
+    return 2 * here <= (S <= 16 ? 5 : 3) * there;
+}
+
+// cols_short_lose, rows of one or two super-blocks in the dot4 layout, of which
+// a round here uses two of eight waves: the dot4 kernels' launches of 8 columns
+// are then ahead of one launch of 16 from 5 (Q4: 7) tiles per CU, of one of 32
+// at 3 launches and of one of 48 from 10, always from 16 (us, dot4 / here:
+// Q6_K 28672 x 512 at 10 / 16 / 24 13.4 / 15.8, 16.5 / 16.0, 23.7 / 20.5; Q4_0
+// 65536 x 512 at 12 / 24 / 32 / 33 18.0 / 21.0, 29.6 / 31.7, 38.3 / 32.6, 44 /
+// 55; 128256 x 512 at 64 107 / 123).
+bool cols_short_lose(double tiles_per_cu, bool q4, int64_t m) {
+    if (tiles_per_cu <= (q4 ? 7 : 5)) return false;
+    return m <= 16 || (tiles_per_cu > 10 && (m <= 24 || (m > 32 && m <= 48))) || tiles_per_cu > 16;
+}
+
+// cols_from_wide, the columns from which rows of S > 32 super-blocks in the
+// dot4 layout come here: 7 where the launch fills the CUs (us, dot4 / here, at
+// 7 and 8: Q4_K 4096 x 14336 21.9 / 20.1 and 28.7 / 19.9, Q6_K 8192 x 14336 44
+// / 40 and 61 / 38, Q8_0 27 / 22.5 and 39 / 22.5); on fewer tiles one round
+// here costs what it costs and the dot4 launch less (1024 x 11008: Q8_0 at 7 /
+// 8 / 9 11.3 / 12.0 / 16.6 against 18.6, Q6_K at 7 / 8 16.3 / 18.1 against
+// 18.6), Q4's excepted up to 64 super-blocks (16.6 / 18.4 against 15.4).
+// Past 64 the dot4 launch takes two (Q6_K 4096 x 20480 at 7 51 / 31).
+int64_t cols_from_wide(const rq_ctx* ctx, const rq_weight* w, int S) {
+    const bool full = w->rows >= 16 * ctx->cus;
+    if (w->fmt == RQ_FMT_Q8_0) return full ? 7 : 10;
+    if (w->fmt == RQ_FMT_Q6_K) return w->rows > 16 * ctx->cus || (full && S > 64) ? 7 : S <= 64 ? 8 : 9;
+    return full || S <= 64 ? 7 : 9;
+}
+
 // Whether m columns of w run the column kernels.
 //   dot4 layout: past the 8 columns of one dot4 launch, each further 8 of
 //     which would read the weights again (us, dot4 / column kernels at 16 and
 //     64 columns: Q4_K 4096 x 4096 17.5 / 7.3 and 69.7 / 15.6, 14336 x 4096
 //     36.7 / 13.7 and 144 / 37.5; Q8_0 11008 x 4096 30.5 / 17.4 and 120 / 44;
 //     Q6_K 4096 x 14336 65 / 20 and 180 / 43, 128256 x 4096 227 / 144 and 894
-//     / 390), but up to two super-blocks on many tiles, of which a round here
-//     uses two of eight waves, at no count (us at 16: Q4_K 65536 x 512 22 / 21,
-//     128256 x 512 32 / 40; Q6_K 28672 x 512 16 / 16, at 10 13.4 / 15.8) and up
-//     to four on the largest not to 12 (128256 x 1024 at 9 37 / 41, at 16 53 /
-//     44). At 8 columns 4096-wide weights are mixed (Q4_K 4096 x 4096 9.3 /
-//     7.3, Q6_K 14336 x 4096 18.7 / 20.4).
+//     / 390), but up to two super-blocks on many tiles where cols_short_lose
+//     says and up to four on the largest not to 12 (128256 x 1024 at 9 37 / 41,
+//     at 16 53 / 44). At 8 columns 4096-wide weights are mixed (Q4_K 4096 x
+//     4096 9.3 / 7.3, Q6_K 14336 x 4096 18.7 / 20.4).
 //     Rows of more than 32 super-blocks, one to a tile there: cols_from_wide.
 //   MFMA layout: Q6_K past 16 columns where q6_cols says, wide rows, which its
 //     16-column class cannot stage, past 8 (4096 x 14336 at 16 / 32 / 64: 22.0
@@ -1115,37 +1158,6 @@ int cols_glu_groups(const rq_ctx* ctx, int fmt, int S) {
 // weights beside it: a group of MFMA-layout weights on both sides runs as two
 // launches (Q4_K 9216 + 2 x 2304 rows of 4096 at 17 columns 30 us, 19.5 when
 // all ran the classes).
-//
-// q6_cols, Q6_K of up to 32 super-blocks in the MFMA layout past 16 columns: by
-// the rounds of one workgroup per CU that either takes, two tiles per
-// workgroup here, 16 waves' worth of k-parts there. A round here costs by its
-// steps of eight super-blocks, about half of one there up to 16 super-blocks
-// and two thirds from 17; below 9 a round there covers up to eight tiles per
-// workgroup at the same cost (us, there / here, at 17 columns: 1024 x 4096
-// 14.9 / 10.3, 8192 x 2048 14.4 / 10.9, 14336 x 4096 27.6 / 27.7, 14336 x 5120
-// 62 / 33, but 12288 x 4608 27.4 / 31.6, 20480 x 2304 25.6 / 32.6, 14336 x 512
-// 9.9 / 13.8, 32000 x 2048 28.3 / 35.6, 128256 x 1024 49 / 96), from four
-// super-blocks on at a little more in the class of 33 to 48 columns (9216 x
-// 2048: 26.0 / 23.1).
-bool q6_cols(const rq_ctx* ctx, int64_t tiles, int S, int64_t m) {
-    const int64_t here = (tiles + 2 * ctx->cus - 1) / (2 * ctx->cus), tr = 16 / ((S + 3) / 4);
-    const int64_t there = (tiles + tr * ctx->cus - 1) / (tr * ctx->cus);
-    return S <= 8 ? here <= there * (S >= 4 && m > 32 && m <= 48 ? 2 : 1) : S <= 16 ? 2 * here <= 5 * there : 2 * here <= 3 * there;
-}
-//
-// cols_from_wide, the columns from which rows of S > 32 super-blocks in the
-// dot4 layout come here: 7 where the launch fills the CUs (us, dot4 / here, at
-// 7 and 8: Q4_K 4096 x 14336 21.9 / 20.1 and 28.7 / 19.9, Q6_K 8192 x 14336 44
-// / 40 and 61 / 38, Q8_0 27 / 22.5 and 39 / 22.5); on fewer tiles one round
-// here costs what it costs and the dot4 launch less (1024 x 11008: Q8_0 at 7 /
-// 8 / 9 11.3 / 12.0 / 16.6 against 18.6, Q6_K at 7 / 8 16.3 / 18.1 against
-// 18.6), Q4's excepted up to 64 super-blocks (16.6 / 18.4 against 15.4).
-int64_t cols_from_wide(const rq_ctx* ctx, const rq_weight* w, int S) {
-    const bool full = w->rows >= 16 * ctx->cus;
-    if (w->fmt == RQ_FMT_Q8_0) return full ? 7 : 10;
-    if (w->fmt == RQ_FMT_Q6_K) return w->rows > 16 * ctx->cus ? 7 : S <= 64 ? 8 : 9;
-    return full || S <= 64 ? 7 : 9;
-}
 bool use_cols(const rq_ctx* ctx, const rq_weight* w, int64_t m) {
     const int S = (int)((w->cols + 255) / 256);
     const bool mfma = use_mmq(w, m);
@@ -1155,7 +1167,8 @@ bool use_cols(const rq_ctx* ctx, const rq_weight* w, int64_t m) {
     if (!mfma && S > 32)
         use = m >= cols_from_wide(ctx, w, S);
     else if (!mfma)
-        use = m > 8 && !(S <= 2 && tiles > (q4 ? 7 : 5) * ctx->cus) && !(S <= 4 && tiles > 16 * ctx->cus && m <= 12);
+        use = m > 8 && !(S <= 2 && cols_short_lose(tiles / (double)ctx->cus, q4, m)) &&
+              !(S <= 4 && tiles > 16 * ctx->cus && m <= 12);
     else if (S > 64 || (S > 32 && w->fmt == RQ_FMT_Q6_K))
         use = m > (S >= 40 || tiles > ctx->cus ? 8 : 16);
     else if (w->fmt == RQ_FMT_Q6_K)
