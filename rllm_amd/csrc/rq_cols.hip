@@ -137,7 +137,6 @@ __device__ __forceinline__ Op fields_op(u32 u0, u32 u1, u32 mask, u32 key, h2 a,
 }
 
 __device__ __forceinline__ _Float16 ubyte_h(u32 w, int i) { return (_Float16)(u16)((w >> (8 * i)) & 0xFFu); }
-__device__ __forceinline__ _Float16 sbyte_h(u32 w, int i) { return (_Float16)(int16_t)(int8_t)(w >> (8 * i)); }
 __device__ __forceinline__ float half_at(u32 w, int i) { return (float)as_h2(w)[i]; }
 
 template <int FMT>
@@ -742,8 +741,9 @@ __device__ __forceinline__ void cols_glu(const RqColsParams& P) {
 #define RQ_COLS_ALL(NAME, FMT)                    \
     RQ_COLS_SET(NAME, FMT, d, RQ_LAY_DOT4)        \
     RQ_COLS(NAME, FMT, d, RQ_LAY_DOT4, 4, 1)      \
-    RQ_COLS(NAME, FMT, d, RQ_LAY_DOT4, 4, 2)      \
     RQ_COLS_SET(NAME, FMT, m, RQ_LAY_MFMA)
+// (4 x 2 of Q8_0 would not fit the LDS.)
+#define RQ_COLS_4X2(NAME, FMT) RQ_COLS(NAME, FMT, d, RQ_LAY_DOT4, 4, 2)
 #define RQ_COLS_GLU(NAME, FMT, CG)                                                                          \
     extern "C" __global__ __launch_bounds__(RQ_COLS_THREADS) void rq_colsglu_##NAME##_##CG(RqColsParams p) { \
         cols_glu<FMT, CG>(p);                                                                               \
@@ -758,6 +758,10 @@ RQ_COLS_FMT(q8_0, RQ_FMT_Q8_0)
 RQ_COLS_FMT(q4_k, RQ_FMT_Q4_K)
 RQ_COLS_FMT(q6_k, RQ_FMT_Q6_K)
 RQ_COLS_ALL(q4_k_q6_k, RQ_FMT_MIX_K)
+RQ_COLS_4X2(q4_0, RQ_FMT_Q4_0)
+RQ_COLS_4X2(q4_k, RQ_FMT_Q4_K)
+RQ_COLS_4X2(q6_k, RQ_FMT_Q6_K)
+RQ_COLS_4X2(q4_k_q6_k, RQ_FMT_MIX_K)
 
 // ---------------------------------------------------------------------------
 // The f16 GEMM route for short prompts (rq_gemm_<fmt>_<layout>): out[a][r] =
@@ -905,14 +909,11 @@ __device__ __forceinline__ void gemm_body(const RqGemmParams& P) {
     const Masks mk = masks<FMT>();
     const int nit = (S + 7) >> 3;
     const int s0 = min(wave, S - 1);
-    // A block's activations are loaded XN - 1 blocks ahead: one block ahead
-    // left each block waiting on an L2 round trip. (Q6_K and Q8_0 in the dot4
-    // layout hold 13 and 17 chunks of the next weights in registers.)
-    constexpr int XN = (LAY == RQ_LAY_DOT4 && ColsFmt<FMT>::C > 9) || CG > 4 ? 2 : 4;
-    Op x[XN][CG];
+    // A block's activations are loaded one block ahead (two to four gained 5 %
+    // at most and lost up to 10, see above).
+    Op x[2][CG];
     Source src;
-#pragma unroll
-    for (int i = 0; i < XN - 1; i++) xload(8 * s0 + i, x[i]);
+    xload(8 * s0, x[0]);
     src.load(C, W, LAY == RQ_LAY_DOT4 ? 0 : s0);
 
     for (int it = 0; it < nit; it++) {
@@ -940,9 +941,9 @@ __device__ __forceinline__ void gemm_body(const RqGemmParams& P) {
             }
 #pragma unroll
             for (int b = 0; b < 4; b++) {
-                const int kb = 8 * s + 4 * hb + b, ahead = 4 * hb + b + XN - 1;
+                const int kb = 8 * s + 4 * hb + b, ahead = 4 * hb + b + 1;
                 // Past the super-block's end: the wave's next one's blocks.
-                xload(ahead < 8 ? 8 * s + ahead : 8 * min(s + 8, S - 1) + ahead - 8, x[ahead % XN]);
+                xload(ahead < 8 ? 8 * s + ahead : 8 * min(s + 8, S - 1) + ahead - 8, x[ahead & 1]);
                 if constexpr (LATE) {
                     if (hb == 0 && b == 0 && it + 1 < nit) src.load(C, W, it + 1);
                     if (b < 3)
@@ -954,7 +955,7 @@ __device__ __forceinline__ void gemm_body(const RqGemmParams& P) {
                 for (int t = 0; t < RT; t++) {
                     const Op o = value_op<FMT, LAY>(h[t], LATE ? u[b & 1][t] : h[t].u[b], b, mk);
 #pragma unroll
-                    for (int c = 0; c < CG; c++) acc[t][c] = mfma(o, x[(4 * hb + b) % XN][c], acc[t][c]);
+                    for (int c = 0; c < CG; c++) acc[t][c] = mfma(o, x[b & 1][c], acc[t][c]);
                 }
             }
             if constexpr (LAY == RQ_LAY_MFMA)

@@ -30,7 +30,7 @@
 
 extern "C" const unsigned char rq_kernels_blob[];  // rq_kernels.hip: Q8_1 pass, dot4 matvecs
 extern "C" const unsigned char rq_mmq_blob[];      // rq_mmq.hip: int8-MFMA matvecs
-extern "C" const unsigned char rq_cols_blob[];     // rq_cols.hip: matvecs over 7 to 64 columns, f16 products
+extern "C" const unsigned char rq_cols_blob[];     // rq_cols.hip: matvecs over more columns (use_cols), f16 products
 // rq_static.hip: the device address of the fixed scratch of
 // rq_matmul_many_noalloc on the current device.
 extern "C" __attribute__((visibility("hidden"))) hipError_t rq_noalloc_scratch(int device, void** ptr, size_t* bytes);
@@ -1002,10 +1002,16 @@ int cols_lds_bytes(int fmt, bool mfma, int rt, int cg, int S) {
     return std::max(stage + x, RQ_COLS_PARTS * rt * cg * 1024);
 }
 
-// Most tiles per workgroup there is a kernel for (more would spill far: of
-// these the 2 x 3 ones of the MFMA layout and the 4 x 2 ones of Q8_0 and Q6_K
-// spill up to 24 registers, which their times below hold).
-int cols_max_rt(bool mfma, int cg) { return cg <= 2 ? (mfma ? 2 : 4) : cg == 3 ? 2 : 1; }
+// Most tiles per workgroup there is a kernel for. (More would spill far. Some
+// of these spill a little, which their times in kColsStep hold, so that the
+// plan takes them only where they are ahead all the same: the MFMA layout's 2 x
+// 3 of Q8_0 24 registers, of Q6_K and the mix 12, 1 x 4 of these 4, the dot4
+// layout's 4 x 2 of these 2 to 3; of the fused gate/up's two groups Q8_0 14 and
+// Q6_K 2. Q8_0's 4 x 2 would not fit the LDS.)
+int cols_max_rt(int fmt, bool mfma, int cg) {
+    if (cg >= 3) return cg == 3 ? 2 : 1;
+    return mfma || (fmt == RQ_FMT_Q8_0 && cg == 2) ? 2 : 4;
+}
 
 // Microseconds of a step (eight super-blocks of the row) in the first and in
 // each further round of workgroups, by layout (dot4, MFMA), type (Q4, Q8_0,
@@ -1016,7 +1022,7 @@ const float kColsStep[2][3][RQ_COLS_MAX_GROUPS][3][2] = {
       {{4.6f, 4.7f}, {6.1f, 6.3f}},
       {{5.9f, 6.0f}}},
      {{{2.4f, 1.6f}, {3.8f, 4.3f}, {6.5f, 7.8f}},
-      {{3.4f, 3.5f}, {5.1f, 5.5f}, {9.5f, 10.5f}},
+      {{3.4f, 3.5f}, {5.1f, 5.5f}},
       {{4.6f, 4.9f}, {6.7f, 7.0f}},
       {{6.0f, 6.3f}}},
      {{{2.6f, 1.6f}, {4.4f, 4.3f}, {7.5f, 8.1f}},
@@ -1061,7 +1067,7 @@ ColsPlan cols_plan(const rq_ctx* ctx, int fmt, bool mfma, int64_t tiles, int S, 
         ColsPlan p;
         p.launches = (m + per - 1) / per;
         p.cg = (int)(((m + p.launches - 1) / p.launches + RQ_COLS_GROUP - 1) / RQ_COLS_GROUP);
-        for (p.rt = 1; p.rt <= cols_max_rt(mfma, p.cg); p.rt *= 2) {
+        for (p.rt = 1; p.rt <= cols_max_rt(fmt, mfma, p.cg); p.rt *= 2) {
             if (cols_lds_bytes(fmt, mfma, p.rt, p.cg, S) > ctx->lds_wide) break;
             const float* step = kColsStep[mfma ? 1 : 0][type][p.cg - 1][p.rt >> 1];
             const int64_t wgs = (tiles + p.rt - 1) / p.rt, rounds = (wgs + ctx->cus - 1) / ctx->cus;
@@ -1692,7 +1698,7 @@ extern "C" rq_status rq_open(int device, rq_ctx** out) {
         const char* fs = f == RQ_NUM_FMTS ? "q4_k_q6_k" : kFmtSuffix[f];
         for (int l = 0; l < 2 && st == RQ_OK; l++)
             for (int cg = 1; cg <= RQ_COLS_MAX_GROUPS && st == RQ_OK; cg++)
-                for (int rt = 1; rt <= cols_max_rt(l == 1, cg) && st == RQ_OK; rt *= 2) {
+                for (int rt = 1; rt <= cols_max_rt(f, l == 1, cg) && st == RQ_OK; rt *= 2) {
                     snprintf(name, sizeof name, "rq_cols_%s_%c_%dx%d", fs, "dm"[l], rt, cg);
                     st = getm(ctx->cols_mod, &ctx->cols[f][l][rt >> 1][cg - 1], name);
                 }
@@ -2931,7 +2937,7 @@ rq_status gated_ffn_run(rq_ctx* ctx, const char* what, const float* x, int64_t x
                     (long long)n);
     if ((st = check_len("gated_ffn gate", gate_len, m * n)) != RQ_OK) return st;
     if ((st = check_len("matmul out", out_len, m * down->rows)) != RQ_OK) return st;
-    if (!glu_fusable(gate, up, m) && !glu_mmq_ok(gate, up, m) && !cols_glu_ok(ctx, gate, up, m) &&
+    if (!glu_fusable(gate, up, m) && !glu_mmq_ok(gate, up, m) &&
         (st = check_len("gated_ffn up", up_len, m * n)) != RQ_OK)
         return st;
     // The f16 GEMM route (f32 x) writes up's product to up_buf when given.

@@ -214,8 +214,8 @@ struct RqMmqParams {
 };
 
 // ---------------------------------------------------------------------------
-// The column kernels (rq_cols_* / rq_colsglu_* in rq_cols.hip): 4 to 64 Q8_1
-// columns against either weight layout.
+// The column kernels (rq_cols_* / rq_colsglu_* in rq_cols.hip): up to 64 Q8_1
+// columns per launch against either weight layout.
 
 // Threads per workgroup: eight waves, wave w taking the super-blocks s of a
 // row with s % 8 == w.
