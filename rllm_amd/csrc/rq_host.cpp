@@ -249,7 +249,7 @@ struct rq_ctx {
     hipFunction_t mmq[RQ_NUM_FMTS + 1][3][3] = {};
     hipFunction_t mmqf[RQ_NUM_FMTS + 1][3] = {};
     hipFunction_t mmqd[RQ_NUM_FMTS][3][3] = {};
-    hipFunction_t mmqg[RQ_NUM_FMTS + 1][4][3] = {};  // 8 x G columns, G = 2, 4 (Q6_K also 6, 8; the mix: 2)
+    hipFunction_t mmqg[RQ_NUM_FMTS + 1][4][3] = {};  // 8 x G columns, G = 2 (Q6_K also 4, 6, 8)
     // 16 x G columns with four-activation entries (Q4_0, Q8_0, Q4_K; G = 1,
     // 2, 4; sbw 2, 4), and the same classes of the fused gate/up (sbw 4)
     hipFunction_t mmqt[RQ_NUM_FMTS][3][2] = {};
@@ -685,7 +685,7 @@ int mmqt_max_cols(int fmt) { return fmt == RQ_FMT_Q6_K ? 16 : 64; }
 // matvec_dispatch.)
 int mmq_max_cols(int fmt, int S2) {
     if (mmq_np(fmt, S2) > 1) return 8;
-    return fmt == RQ_FMT_MIX_K ? 16 : mmq_has_t(fmt, S2) || fmt == RQ_FMT_Q6_K ? 64 : 32;
+    return fmt == RQ_FMT_MIX_K ? 16 : mmq_has_t(fmt, S2) || fmt == RQ_FMT_Q6_K ? 64 : 16;
 }
 // Table index of an 8 x g class.
 int mmqg_index(int g) { return g == 2 ? 0 : g == 4 ? 1 : g == 6 ? 2 : 3; }
@@ -1631,7 +1631,7 @@ extern "C" rq_status rq_open(int device, rq_ctx** out) {
             snprintf(name, sizeof name, "rq_mmqf_%s_%d", kFmtSuffix[f], kMmqSbw[si]);
             st = getm(ctx->mmq_mod, &ctx->mmqf[f][si], name);
             for (int gi = 0; gi < 4 && st == RQ_OK; gi++) {
-                if (gi >= 2 && (f != RQ_FMT_Q6_K || kMmqSbw[si] != 4)) continue;  // 8 x 6, 8 x 8: Q6_K only
+                if (gi >= 1 && (f != RQ_FMT_Q6_K || (gi >= 2 && kMmqSbw[si] != 4))) continue;  // 8 x 4 to 8 x 8: Q6_K
                 snprintf(name, sizeof name, "rq_mmq_%s_8x%d_%d", kFmtSuffix[f], 2 * (gi + 1), kMmqSbw[si]);
                 st = getm(ctx->mmq_mod, &ctx->mmqg[f][gi][si], name);
             }
@@ -1648,6 +1648,7 @@ extern "C" rq_status rq_open(int device, rq_ctx** out) {
     for (int f = 0; f < RQ_NUM_FMTS && st == RQ_OK; f++) {
         for (int gi = 0; gi < (f == RQ_FMT_Q6_K ? 1 : 3) && st == RQ_OK; gi++) {  // Q6_K: 16 x 1, sbw 4 only
             for (int si = f == RQ_FMT_Q6_K ? 1 : 0; si < 2 && st == RQ_OK; si++) {
+                if (gi > 0 && si == 1 && f != RQ_FMT_Q4_K) continue;  // (rq_cols_* there)
                 snprintf(name, sizeof name, "rq_mmq_%s_16x%d_%d", kFmtSuffix[f], 1 << gi, kMmqSbw[si]);
                 st = getm(ctx->mmq_mod, &ctx->mmqt[f][gi][si], name);
             }

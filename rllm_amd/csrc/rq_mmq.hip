@@ -1610,7 +1610,6 @@ __device__ __forceinline__ void mmq_run(const RqMmqParams& P) {
     RQ_MMQ(NAME, FMT, 4, SBW)                                                                    \
     RQ_MMQ(NAME, FMT, 8, SBW)                                                                    \
     RQ_MMQ_G(NAME, FMT, 2, SBW)                                                                  \
-    RQ_MMQ_G(NAME, FMT, 4, SBW)                                                                  \
     extern "C" __global__ __launch_bounds__(1024) void rq_mmqf_##NAME##_##SBW(RqMmqParams p) {     \
         mmq_run<FMT, 1, SBW, true, false>(p);                                                    \
     }
@@ -1635,6 +1634,9 @@ extern "C" __global__ __launch_bounds__(512) void rq_mmq_q6_k_1_8(RqMmqParams p)
 extern "C" __global__ __launch_bounds__(512) void rq_mmqf_q6_k_8(RqMmqParams p) {
     mmq_run<RQ_FMT_Q6_K, 1, 8, true, false>(p);
 }
+// 17 to 64 columns of Q6_K (the other formats run 16-column classes there).
+RQ_MMQ_G(q6_k, RQ_FMT_Q6_K, 4, 2)
+RQ_MMQ_G(q6_k, RQ_FMT_Q6_K, 4, 4)
 RQ_MMQ_G(q6_k, RQ_FMT_Q6_K, 6, 4)
 RQ_MMQ_G(q6_k, RQ_FMT_Q6_K, 8, 4)
 // Fused gate/up + activation + Q8_1 of the product (the reference's
@@ -1731,9 +1733,9 @@ RQ_MMQ_GLU_WIDE(q6_k, RQ_FMT_Q6_K)
     extern "C" __global__ __launch_bounds__(1024) void rq_mmq_##NAME##_16x##G##_##SBW(RqMmqParams p) {       \
         mmqt_body<FMT, SBW, G, false>(p);                                                                   \
     }
+// (Past 16 columns rows of more than 16 super-blocks run rq_cols_*: 4
+// super-blocks per wave are then Q4_K's alone, of more than 512 tiles.)
 #define RQ_MMQT_SET(NAME, FMT, G)                                                                          \
-    RQ_MMQT(NAME, FMT, G, 2)                                                                               \
-    RQ_MMQT(NAME, FMT, G, 4)                                                                               \
     extern "C" __global__ __launch_bounds__(1024) void rq_mmqglu_##NAME##_16x##G(RqMmqParams p) {           \
         mmqt_body<FMT, 4, G, true>(p);                                                                      \
     }
@@ -1744,6 +1746,16 @@ RQ_MMQ_GLU_WIDE(q6_k, RQ_FMT_Q6_K)
 RQ_MMQT_FMT(q4_0, RQ_FMT_Q4_0)
 RQ_MMQT_FMT(q8_0, RQ_FMT_Q8_0)
 RQ_MMQT_FMT(q4_k, RQ_FMT_Q4_K)
+#define RQ_MMQT_16(NAME, FMT) \
+    RQ_MMQT(NAME, FMT, 1, 2)  \
+    RQ_MMQT(NAME, FMT, 1, 4)  \
+    RQ_MMQT(NAME, FMT, 2, 2)  \
+    RQ_MMQT(NAME, FMT, 4, 2)
+RQ_MMQT_16(q4_0, RQ_FMT_Q4_0)
+RQ_MMQT_16(q8_0, RQ_FMT_Q8_0)
+RQ_MMQT_16(q4_k, RQ_FMT_Q4_K)
+RQ_MMQT(q4_k, RQ_FMT_Q4_K, 2, 4)
+RQ_MMQT(q4_k, RQ_FMT_Q4_K, 4, 4)
 // Q6_K: one group of 16 (a second group would need its 66 registers of
 // weights held across groups, and spills), 4 super-blocks per wave.
 #define RQ_MMQT6(G)                                                                                        \
