@@ -1018,10 +1018,10 @@ int cols_max_rt(int fmt, bool mfma, int cg) {
 // Q6_K), column groups and log2 of the tiles per workgroup (0: no kernel).
 const float kColsStep[2][3][RQ_COLS_MAX_GROUPS][3][2] = {
     {{{{2.1f, 1.3f}, {3.2f, 2.0f}, {5.4f, 6.0f}},
-      {{3.3f, 3.3f}, {4.5f, 4.7f}, {7.0f, 7.8f}},
+      {{3.3f, 3.3f}, {4.5f, 4.7f}, {7.5f, 8.0f}},
       {{4.6f, 4.7f}, {6.1f, 6.3f}},
       {{5.9f, 6.0f}}},
-     {{{2.4f, 1.6f}, {3.8f, 4.3f}, {6.5f, 7.8f}},
+     {{{2.4f, 1.6f}, {4.3f, 4.4f}, {6.5f, 7.8f}},
       {{3.4f, 3.5f}, {5.1f, 5.5f}},
       {{4.6f, 4.9f}, {6.7f, 7.0f}},
       {{6.0f, 6.3f}}},
@@ -1053,15 +1053,16 @@ const float kColsStep[2][3][RQ_COLS_MAX_GROUPS][3][2] = {
 // layout, at 17 / 64 columns 17.6 / 28.9 us against 13.4 / 24.6 at two; Q8_0
 // 14336 x 4096, dot4, at 24 45 us at four against 28.) Measured over 15 sizes
 // from 96 to 128256 rows, 512 to 14336 columns and 9 to 64 tokens (13404
-// calls): the choice is within 5 % of the best in 97 %, within 14 % in all.
+// calls): the choice is within 5 % of the best in 97 %, within 14 % in all. (A
+// mixed launch is priced as the type that most of its tiles have.)
 struct ColsPlan {
     int rt = 0, cg = 0;
     int64_t launches = 0;
 };
-ColsPlan cols_plan(const rq_ctx* ctx, int fmt, bool mfma, int64_t tiles, int S, int64_t m) {
+ColsPlan cols_plan(const rq_ctx* ctx, int fmt, bool mfma, int64_t tiles, int64_t q6_tiles, int S, int64_t m) {
     ColsPlan best;
     double best_us = 0;
-    const int type = fmt == RQ_FMT_Q8_0 ? 1 : fmt == RQ_FMT_Q6_K || fmt == RQ_FMT_MIX_K ? 2 : 0, steps = (S + 7) / 8;
+    const int type = fmt == RQ_FMT_Q8_0 ? 1 : 2 * q6_tiles > tiles ? 2 : 0, steps = (S + 7) / 8;
     for (int max_cg = RQ_COLS_MAX_GROUPS; max_cg >= 1; max_cg--) {
         const int64_t per = RQ_COLS_GROUP * max_cg;
         ColsPlan p;
@@ -1069,9 +1070,15 @@ ColsPlan cols_plan(const rq_ctx* ctx, int fmt, bool mfma, int64_t tiles, int S, 
         p.cg = (int)(((m + p.launches - 1) / p.launches + RQ_COLS_GROUP - 1) / RQ_COLS_GROUP);
         for (p.rt = 1; p.rt <= cols_max_rt(fmt, mfma, p.cg); p.rt *= 2) {
             if (cols_lds_bytes(fmt, mfma, p.rt, p.cg, S) > ctx->lds_wide) break;
-            const float* step = kColsStep[mfma ? 1 : 0][type][p.cg - 1][p.rt >> 1];
             const int64_t wgs = (tiles + p.rt - 1) / p.rt, rounds = (wgs + ctx->cus - 1) / ctx->cus;
-            const double us = p.launches * (3.2 + step[0] * steps + (rounds - 1) * (1.0 + step[1] * steps));
+            const int64_t low = m / p.launches, more = m % p.launches;  // `more` launches of low + 1 columns
+            double us = 0;
+            for (int i = 0; i < 2; i++) {
+                const int64_t count = i ? more : p.launches - more, cg = (low + i + RQ_COLS_GROUP - 1) / RQ_COLS_GROUP;
+                if (count == 0) continue;
+                const float* step = kColsStep[mfma ? 1 : 0][type][cg - 1][p.rt >> 1];
+                us += count * (3.2 + step[0] * steps + (rounds - 1) * (1.0 + step[1] * steps));
+            }
             if (best.rt == 0 || us < best_us) best = p, best_us = us;
         }
     }
@@ -1097,10 +1104,10 @@ int cols_glu_groups(const rq_ctx* ctx, int fmt, int S) {
 // 9.9 / 13.8, 32000 x 2048 28.3 / 35.6, 128256 x 1024 49 / 96), from four
 // super-blocks on at a little more in the class of 33 to 48 columns (9216 x
 // 2048: 26.0 / 23.1).
-bool q6_cols(const rq_ctx* ctx, int64_t tiles, int S, int64_t m) {
+bool q6_cols(const rq_ctx* ctx, int64_t tiles, int S, int64_t per) {
     const int64_t here = (tiles + 2 * ctx->cus - 1) / (2 * ctx->cus), tr = 16 / ((S + 3) / 4);
     const int64_t there = (tiles + tr * ctx->cus - 1) / (tr * ctx->cus);
-    if (S <= 8) return here <= there * (S >= 4 && m > 32 && m <= 48 ? 2 : 1);
+    if (S <= 8) return here <= there * (S >= 4 && per > 32 && per <= 48 ? 2 : 1);
     return 2 * here <= (S <= 16 ? 5 : 3) * there;
 }
 
@@ -1155,8 +1162,8 @@ int64_t cols_from_wide(const rq_ctx* ctx, const rq_weight* w, int S) {
 //     175 / 126), of shorter rows up to two tiles per CU (Q4_K 4096 x 4096 at
 //     32 / 48 / 64: 10.9 / 17.8 / 19.0 -> 9.3 / 11.9 / 15.0 us), above which
 //     the classes read the activations for four tiles at once (14336 x 4096
-//     at 32: 18.9 against 22.4 us). Past 48 columns two tiles per workgroup
-//     take two launches here, which cost the classes' four-fold staging of
+//     at 32: 18.9 against 22.4 us). Past 48 columns a launch two tiles per
+//     workgroup take two launches here, which cost the classes' four-fold staging of
 //     Q8_0's rows up to 9 super-blocks, and of the others' from 13 (Q8_0 8192
 //     x 1024 at 64 14.6 / 16.8, Q4_K 8192 x 4096 22.9 / 25.2; between, Q4_K
 //     8192 x 3072 26.2 / 22.0).
@@ -1170,6 +1177,7 @@ bool use_cols(const rq_ctx* ctx, const rq_weight* w, int64_t m) {
     bool use;
     const int64_t tiles = (w->rows + 15) / 16;
     const bool q4 = w->fmt == RQ_FMT_Q4_K || w->fmt == RQ_FMT_Q4_0;
+    const int64_t per = (m + (m + 63) / 64 - 1) / ((m + 63) / 64);  // columns of a launch of the classes
     if (!mfma && S > 32)
         use = m >= cols_from_wide(ctx, w, S);
     else if (!mfma)
@@ -1178,11 +1186,11 @@ bool use_cols(const rq_ctx* ctx, const rq_weight* w, int64_t m) {
     else if (S > 64 || (S > 32 && w->fmt == RQ_FMT_Q6_K))
         use = m > (S >= 40 || tiles > ctx->cus ? 8 : 16);
     else if (w->fmt == RQ_FMT_Q6_K)
-        use = m > 16 && q6_cols(ctx, tiles, S, m);
+        use = m > 16 && q6_cols(ctx, tiles, S, per);
     else
         use = m > 16 && (S > 16 || (tiles <= 2 * ctx->cus &&
-                                    (m <= 48 || tiles <= ctx->cus || (w->fmt == RQ_FMT_Q8_0 ? S > 9 : S <= 12))));
-    return use && cols_plan(ctx, w->fmt, mfma, 1, S, m).rt > 0;
+                                    (per <= 48 || tiles <= ctx->cus || (w->fmt == RQ_FMT_Q8_0 ? S > 9 : S <= 12))));
+    return use && cols_plan(ctx, w->fmt, mfma, 1, 0, S, m).rt > 0;
 }
 
 int log2_of(int v) {
@@ -1219,14 +1227,15 @@ rq_status cols_launch(rq_ctx* ctx, const int8_t* xq, const uint16_t* xd, int64_t
                       float* const* outs, int count) {
     const bool mfma = use_mmq(ws[0], m);
     int fmt = ws[0]->fmt;
-    int64_t tiles = 0;
+    int64_t tiles = 0, q6_tiles = 0;
     for (int i = 0; i < count; i++) {
         if (ws[i]->fmt != fmt) fmt = RQ_FMT_MIX_K;
         tiles += (ws[i]->rows + 15) / 16;
+        if (ws[i]->fmt == RQ_FMT_Q6_K) q6_tiles += (ws[i]->rows + 15) / 16;
     }
     const int64_t k = ws[0]->cols;
     const int S = (int)((k + 255) / 256);
-    const ColsPlan plan = cols_plan(ctx, fmt, mfma, tiles, S, m);
+    const ColsPlan plan = cols_plan(ctx, fmt, mfma, tiles, q6_tiles, S, m);
     if (plan.rt == 0) return fail(RQ_ERR_SHAPE, "matvec: %lld columns too wide to stage", (long long)k);
     const int rt = plan.rt;
     for (int64_t gi = 0, g0 = 0; gi < plan.launches; gi++) {
