@@ -171,8 +171,9 @@ def bench_matvec(torch, gpu, orc, t, n, k, m, steps, warmup, seed=7, family=None
 def bench_matmul_routes(torch, gpu, orc, t, n, k, m, steps, warmup, seed=7):
     """rq_matmul at m columns from f32 inputs, both routes of a batched
     matmul on MFMA-layout weights rotating over copies: the int8 path
-    (activations to Q8_1, int8 MFMA) and the f16 GEMM route (activations and
-    weights to f16, rocBLAS gemm_ex with f32 output), each forced with
+    (activations to Q8_1, int8-MFMA or column kernels) and the f16 GEMM route
+    (activations and weights to f16, own kernels or rocBLAS gemm_ex, with f32
+    output), each forced with
     rq_set_gemm_min_m whatever the default would pick, and the route again
     on weights that keep a persistent f16 copy (rq_weight_keep_f16: no
     dequantization in the call). Returns {route:

@@ -266,7 +266,7 @@ class HipBackend:
         m == 1: each launch quantizes x while staging it; m >= 2: x is
         quantized once into the context's scratch (see reserve). From
         GEMM_MIN_M_DEFAULT columns (set_gemm_min_m): the f16 GEMM route,
-        x and each weight in f16, rocBLAS with f32 output (see reserve_f16)."""
+        x and each weight in f16, f32 output (see reserve_f16)."""
         if len(ws) != len(outs) or not ws:
             raise ShapeError(f"matmul_many: {len(ws)} weights, {len(outs)} outputs")
         _lib.check(_lib.lib().rq_matmul_many(self.ctx, x.data_ptr(), x.numel(), m, _ptrs([w.handle for w in ws]),

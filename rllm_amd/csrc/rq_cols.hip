@@ -1,11 +1,12 @@
-// Matvecs over more than 8 activation columns (rq_cols_*, either weight
-// layout, rq_params.h) and the fused gate/up front half of a gated FFN
-// (rq_colsglu_*, the dot4 layout); on the same weight sources the f16 GEMM
-// route's kernels for short prompts (rq_gemm_*, at the end). Which calls come
+// Matvecs over more activation columns than the dot4 kernels or the int8-MFMA
+// classes do best (rq_cols_*, either weight layout, rq_params.h) and the fused
+// gate/up front half of a gated FFN (rq_colsglu_*, the dot4 layout); on the
+// same weight sources the f16 GEMM route's kernels for short prompts
+// (rq_gemm_*, at the end). Which calls come
 // here, and both sides' times: use_cols and gemm_fused in rq_host.cpp.
 //
 // What bounds them. Every weight is read once, so a launch cannot be faster
-// than its bytes; up to about 16 columns that is the bound. The work beside
+// than its bytes, which none is close to (counters below). The work beside
 // it is per (row, 32-element block, column): the block's exact dot has to be
 // scaled by the activation block's own scale before it is summed. With
 // int8 MFMAs (K = 64, two blocks) that took half-empty operands and three
@@ -40,13 +41,14 @@
 //
 // Measured (us, replayed launches over weights beyond the caches; before:
 // the dot4 kernels in groups of 8 columns, the int8-MFMA classes):
-//   Q4_K 4096 x 4096, dot4 layout, 16 / 64 columns    17.5 / 69.7 -> 7.3 / 15.6
-//   Q4_K 14336 x 4096, dot4 layout, 16 / 32           36.7 / 73.1 -> 13.7 / 18.7
-//   Q6_K 4096 x 14336, MFMA layout, 16 / 32 / 64      22.0 / 37.9 / 72.9 -> 17.9 / 25.3 / 42.9
-//   Q4_K q, k and Q6_K v of width 5120, dot4, 43      206 -> 41 (one launch for six)
-// At 14336 x 4096 and 16 columns the launch reads its 33 MB at 2.4 TB/s: 30
-// VALU per operand and column group, 54% of the issue slots of its 8 waves
-// per CU; the rest is the first loads' latency (one step in flight) and LDS.
+//   Q4_K 4096 x 4096, dot4 layout, 16 / 64 columns    17.6 / 70.2 -> 7.5 / 16.4
+//   Q4_K 14336 x 4096, dot4 layout, 16 / 32           36.7 / 73.0 -> 15.7 / 20.2
+//   Q6_K 4096 x 14336, MFMA layout, 16 / 32 / 64      21.7 / 37.7 / 72.8 -> 18.5 / 25.7 / 42.9
+//   Q4_K q, k and Q6_K v of width 5120, dot4, 43      211 -> 46 (one launch for six, and the Q8_1 pass)
+// Counters of 14336 x 4096 at 16 columns, dot4 layout: 3.87 M VALU
+// instructions, 44% of the issue cycles of the CUs that hold a workgroup (Q6_K
+// 4096 x 14336 at 32, MFMA layout: 51%), MFMA busy 9 to 13%; the rest is the
+// loads' latency (one step in flight, one workgroup per CU) and LDS.
 
 #include "rq_device.h"
 
@@ -777,8 +779,9 @@ RQ_COLS_4X2(q4_k_q6_k, RQ_FMT_MIX_K)
 // fewer columns per workgroup would dequantize more than they multiply, and
 // more rows would leave the chip short of workgroups (64 rows by 64 columns:
 // 14336 x 4096 at 128 columns 45 us against 38). What is left is bound by the
-// reads of x, 1 KB per wave and two products (448 MB from L2 for 14336 x 4096
-// at 128 columns, 12 TB/s), not by VALU or by the loads in flight: 16 % fewer
+// reads of x, 1 KB per wave and two products (510 MB of reads from L2 for 14336
+// x 4096 at 128 columns, 14 TB/s, by counters; VALU issue 27%, MFMA busy 17%),
+// not by VALU or by the loads in flight: 16 % fewer
 // VALU instructions took 1 to 3 % off some shapes and put as much on others
 // (128 columns 36.5 -> 35.9 us, 96 30.6 -> 31.4), and loads two to four
 // blocks ahead on top gained 5 % at most (Q6_K 4096 x 14336 at 128: 57.4 ->

@@ -1141,17 +1141,17 @@ int64_t cols_from_wide(const rq_ctx* ctx, const rq_weight* w, int S) {
 // Whether m columns of w run the column kernels.
 //   dot4 layout: past the 8 columns of one dot4 launch, each further 8 of
 //     which would read the weights again (us, dot4 / column kernels at 16 and
-//     64 columns: Q4_K 4096 x 4096 17.5 / 7.3 and 69.7 / 15.6, 14336 x 4096
-//     36.7 / 13.7 and 144 / 37.5; Q8_0 11008 x 4096 30.5 / 17.4 and 120 / 44;
-//     Q6_K 4096 x 14336 65 / 20 and 180 / 43, 128256 x 4096 227 / 144 and 894
+//     64 columns: Q4_K 4096 x 4096 17.6 / 7.5 and 70.2 / 16.4, 14336 x 4096
+//     36.7 / 15.7 and 144 / 39.9; Q8_0 11008 x 4096 30.2 / 17.8 and 118 / 43;
+//     Q6_K 4096 x 14336 65 / 21 and 179 / 43, 128256 x 4096 227 / 144 and 894
 //     / 390), but up to two super-blocks on many tiles where cols_short_lose
 //     says and up to four on the largest not to 12 (128256 x 1024 at 9 37 / 41,
 //     at 16 53 / 44). At 8 columns 4096-wide weights are mixed (Q4_K 4096 x
 //     4096 9.3 / 7.3, Q6_K 14336 x 4096 18.7 / 20.4).
 //     Rows of more than 32 super-blocks, one to a tile there: cols_from_wide.
 //   MFMA layout: Q6_K past 16 columns where q6_cols says, wide rows, which its
-//     16-column class cannot stage, past 8 (4096 x 14336 at 16 / 32 / 64: 22.0
-//     / 37.9 / 72.9 -> 17.9 / 25.3 / 42.9 us), but below 40 super-blocks on no
+//     16-column class cannot stage, past 8 (4096 x 14336 at 16 / 32 / 64: 21.7
+//     / 37.7 / 72.8 -> 18.5 / 25.7 / 42.9 us), but below 40 super-blocks on no
 //     more tiles than CUs past 16 (4096 x 8448 at 9 / 16 12.2 / 13.4 in the
 //     classes, 14.3 / 13.8 here); past 64 super-blocks every type, whose
 //     classes stop at 8 columns there;
@@ -1160,7 +1160,7 @@ int64_t cols_from_wide(const rq_ctx* ctx, const rq_weight* w, int S) {
 //     / here, at 17 and 64 columns: Q4_K 4096 x 5120 13.7 / 12.3 and 25.1 /
 //     19.0, 14336 x 5120 33.8 / 28.5 and 64 / 53, Q8_0 28672 x 6144 87 / 66 and
 //     175 / 126), of shorter rows up to two tiles per CU (Q4_K 4096 x 4096 at
-//     32 / 48 / 64: 10.9 / 17.8 / 19.0 -> 9.3 / 11.9 / 15.0 us), above which
+//     32 / 48 / 64: 10.9 / 17.8 / 19.1 -> 9.6 / 12.5 / 15.6 us), above which
 //     the classes read the activations for four tiles at once (14336 x 4096
 //     at 32: 18.9 against 22.4 us). Past 48 columns a launch two tiles per
 //     workgroup take two launches here, which cost the classes' four-fold staging of

@@ -55,10 +55,8 @@ def test_mmq_column_classes(mfma, orc, tname, m):
 
 @pytest.mark.parametrize("m", [33, 40, 48, 57, 64])
 def test_mmq_q6_k_wide_rows_many_columns(mfma, orc, m):
-    """Q6_K ffn_down's width (k = 14336) at 33 to 64 columns: one launch of
-    the 8 x 6 / 8 x 8 classes, which add each group's k-parts as it ends
-    (8 staged columns of this width leave no LDS for every group's partial
-    sums)."""
+    """Q6_K ffn_down's width (k = 14336) at 33 to 64 columns: one launch of the
+    column kernels (the 8 x 6 / 8 x 8 classes: test_gpu_cols.py)."""
     _run(mfma, orc, MMQ_TYPES["Q6_K"], 35, 14336, m, 14336 + m, kind="normal")
 
 
